@@ -1249,4 +1249,112 @@ int qd_batch_gemv(const float* x, long ldx, const void* gamma, float eps, const 
   return qd::gemv8_launch(g, qd::EPI_STORE, S(stream));
 }
 
+// ---------------------------------------------------------------- prefill
+
+namespace {
+
+struct PrefillBuffers {
+  size_t h, img, scale, o_scale, part, cs, q_img, k_img, vt_img, vexp, vmax, argmax;
+};
+
+// Workspace of a prefill of S rows, or 0 where the kernels do not apply.
+size_t prefill_layout(const qd_model_desc* d, long S_, qd::PrefillPlan* plan, PrefillBuffers* b) {
+  const long H = d->hidden, I = d->intermediate, Hq = d->num_heads, Hkv = d->num_kv_heads;
+  const bool fixed_k = H == 512 || H == 1024 || H == 2048 || H == 3072 || H == 4096 || H == 6144;
+  if (batch_of(d) > 1 || d->num_layers < 1 || d->head_dim != 128 || !fixed_k || I < 512 || I % 512 != 0 || I > 16384 ||
+      Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || Hq * 128 % 512 != 0 || d->vocab < 1 || S_ < 1)
+    return 0;
+  const long qs = Hq * 128, qn = qs + 2 * Hkv * 128;
+  const long kmax = std::max(H, std::max(qs, I)), nmax = std::max(2 * I, qn);
+  // 32-bit byte offsets into the GEMM operands
+  if ((kmax * S_ * 2) >> 32 || (nmax * kmax * 2) >> 32 || S_ * (Hq + Hkv) >> 31) return 0;
+  *plan = qd::prefill_plan(S_, (int)H, (int)Hq, (int)Hkv, (int)I);
+  if (plan->qkv.tile < 0 || plan->o_proj.tile < 0 || plan->gate_up.tile < 0 || plan->down.tile < 0) return 0;
+  const long tiles = (S_ + 63) / 64;
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    const size_t o = off;
+    off += align256(n);
+    return o;
+  };
+  b->h = take(4 * (size_t)S_ * H);
+  b->img = take(4 * (size_t)S_ * kmax);
+  b->scale = take(4 * (size_t)S_);
+  b->o_scale = take(4);
+  b->part = take(4 * (size_t)plan->part_floats);
+  b->cs = take(8 * (size_t)S_ * 64);
+  b->q_img = take(4 * (size_t)S_ * qs);
+  b->k_img = take(4 * (size_t)S_ * Hkv * 128);
+  b->vt_img = take(4 * (size_t)tiles * 64 * Hkv * 128);
+  b->vexp = take(4 * (size_t)tiles * Hkv);
+  b->vmax = take(4 * (size_t)d->num_layers);
+  b->argmax = take(argmax_ws_bytes());
+  return off;
+}
+
+}  // namespace
+
+size_t qd_prefill_workspace_bytes(const qd_model_desc* d, int rows) {
+  if (d == nullptr) return 0;
+  qd::PrefillPlan plan;
+  PrefillBuffers b;
+  return prefill_layout(d, rows, &plan, &b);
+}
+
+int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int n_vision, const int64_t* text_ids,
+               const int64_t* position_ids, int rows, int64_t* token_out, void* workspace, size_t workspace_bytes,
+               void* stream) {
+  QD_REQUIRE(d && d->layers && d->embed && d->final_norm && d->inv_freq && position_ids && token_out && workspace,
+             QD_ERR_ARG, "null pointer");
+  QD_REQUIRE(vision_dtype == QD_F16 || vision_dtype == QD_F32, QD_ERR_ARG, "bad vision dtype");
+  QD_REQUIRE(rows >= 1 && n_vision >= 0 && n_vision <= rows && rows <= d->capacity, QD_ERR_SHAPE,
+             "need 0 <= n_vision <= rows <= capacity (n_vision=%d rows=%d capacity=%d)", n_vision, rows, d->capacity);
+  QD_REQUIRE((n_vision == 0 || (vision && a16(vision))) && (n_vision == rows || text_ids), QD_ERR_ARG,
+             "missing or misaligned prompt rows");
+  qd::PrefillPlan plan;
+  PrefillBuffers b;
+  const size_t need = prefill_layout(d, rows, &plan, &b);
+  QD_REQUIRE(need > 0, QD_ERR_SHAPE, "prefill needs head_dim 128, H in {512, 1024, 2048, 3072, 4096, 6144}, I %% 512 == 0, "
+             "Hq %% Hkv == 0 and batch 1");
+  QD_REQUIRE(workspace_bytes >= need && aligned(workspace, 256), QD_ERR_WORKSPACE,
+             "workspace of %zu bytes, 256-byte aligned (got %zu)", need, workspace_bytes);
+  QD_REQUIRE(a16(d->embed) && a16(d->final_norm), QD_ERR_ARG, "weights must be 16-byte aligned");
+  std::vector<qd::PrefillLayer> layers((size_t)d->num_layers);
+  for (int i = 0; i < d->num_layers; ++i) {
+    const qd_layer_weights& w = d->layers[i];
+    QD_REQUIRE(w.qkv && w.o_proj && w.gate_up && w.down && w.input_norm && w.post_norm && w.q_norm && w.k_norm &&
+                   w.k_cache && w.v_cache,
+               QD_ERR_ARG, "layer %d: null pointer", i);
+    QD_REQUIRE(a16(w.qkv) && a16(w.o_proj) && a16(w.gate_up) && a16(w.down) && a16(w.input_norm) && a16(w.post_norm),
+               QD_ERR_ARG, "layer %d: weights must be 16-byte aligned", i);
+    layers[(size_t)i] = qd::PrefillLayer{(const u16*)w.qkv,        (const u16*)w.o_proj,    (const u16*)w.gate_up,
+                                         (const u16*)w.down,       (const u16*)w.input_norm, (const u16*)w.post_norm,
+                                         (const u16*)w.q_norm,     (const u16*)w.k_norm,    (u16*)w.k_cache,
+                                         (u16*)w.v_cache};
+  }
+  char* base = reinterpret_cast<char*>(workspace);
+  qd::PrefillArgs a;
+  a.S = rows; a.layers_n = d->num_layers; a.H = d->hidden; a.Hq = d->num_heads; a.Hkv = d->num_kv_heads;
+  a.I = d->intermediate; a.T = d->capacity; a.eps = d->eps; a.attn_scale = 1.0f / sqrtf((float)d->head_dim);
+  a.sec_h = d->sec_h; a.sec_w = d->sec_w; a.inv_freq = d->inv_freq; a.embed = (const u16*)d->embed;
+  a.vision = vision; a.vision_f32 = vision_dtype == QD_F32; a.n_vision = n_vision; a.text_ids = text_ids;
+  a.position_ids = position_ids;
+  a.h = reinterpret_cast<float*>(base + b.h);
+  a.img = reinterpret_cast<u16*>(base + b.img);
+  a.scale = reinterpret_cast<float*>(base + b.scale);
+  a.o_scale = reinterpret_cast<float*>(base + b.o_scale);
+  a.part = reinterpret_cast<float*>(base + b.part);
+  a.cs = reinterpret_cast<float2*>(base + b.cs);
+  a.q_img = reinterpret_cast<u16*>(base + b.q_img);
+  a.k_img = reinterpret_cast<u16*>(base + b.k_img);
+  a.vt_img = reinterpret_cast<u16*>(base + b.vt_img);
+  a.vexp = reinterpret_cast<int*>(base + b.vexp);
+  a.vmax = reinterpret_cast<int*>(base + b.vmax);
+  a.argmax_count = reinterpret_cast<unsigned*>(base + b.argmax);
+  const int st = qd::prefill_launch(a, layers.data(), plan, S(stream));
+  if (st) return st;
+  return qd_lm_head_argmax(a.h + (size_t)(rows - 1) * d->hidden, QD_F32, d->final_norm, d->eps, d->embed, d->vocab,
+                           d->hidden, nullptr, token_out, base + b.argmax, stream);
+}
+
 }  // extern "C"

@@ -314,4 +314,64 @@ int advance8_launch(const int64_t* token, int64_t* out_tokens, int64_t* counter,
 // 0 when the device can keep the whole persistent grid resident at once.
 int decode_persistent_check_device(char* why, size_t why_len);
 
+// ---------------------------------------------------------------- prefill
+
+// y[z][M][N] = scale[m * scale_stride] * (hi + lo)[M][K] . W[N][K]^T over K
+// range z of the plan (fp16 operands, fp32 accumulation).  N % 4 == 0, K a
+// multiple of the plan's tile depth times z, operands below 4 GB each.
+struct SplitGemmArgs {
+  const uint16_t* hi = nullptr;   // fp16 [M][K]
+  const uint16_t* lo = nullptr;   // fp16 [M][K]
+  const float* scale = nullptr;
+  int scale_stride = 1;           // 1: one scale per row; 0: one for all rows
+  const uint16_t* W = nullptr;    // fp16 [N][K]
+  float* y = nullptr;             // fp32 [z][M][N]
+  int M = 0, N = 0, K = 0;
+};
+struct GemmPlan {
+  int tile;   // index of the tile shape
+  int z;      // K ranges, one workgroup and one output plane each
+};
+constexpr int kPrefillMaxSplit = 16;
+GemmPlan split_gemm_plan(long M, long N, long K);
+int split_gemm_launch(const SplitGemmArgs& a, const GemmPlan& p, hipStream_t s);
+
+struct PrefillLayer {
+  const uint16_t *qkv, *o_proj, *gate_up, *down, *input_norm, *post_norm, *q_norm, *k_norm;
+  uint16_t *k_cache, *v_cache;
+};
+
+// One prefill of S rows: the prompt (n_vision embedding rows, then token ids),
+// the positions and the workspace buffers.
+struct PrefillArgs {
+  int S, layers_n, H, Hq, Hkv, I, T;
+  float eps, attn_scale;
+  int sec_h, sec_w;
+  const float* inv_freq;          // fp32 [64]
+  const uint16_t* embed;          // fp16 [V][H]
+  const void* vision;             // fp16 or fp32 [n_vision][H]
+  int vision_f32, n_vision;
+  const int64_t* text_ids;        // [S - n_vision]
+  const int64_t* position_ids;    // [3][S]
+  float* h;                       // [S][H] residual stream
+  uint16_t* img;                  // split image (hi plane, lo plane) of the next GEMM's input
+  float* scale;                   // [S] its row scales
+  float* o_scale;                 // [1] scale of the attention output's image
+  float* part;                    // GEMM output planes
+  float2* cs;                     // [S][64] cos, sin
+  uint16_t* q_img;                // 2 x [Hq][S][128]
+  uint16_t* k_img;                // 2 x [Hkv][S][128]
+  uint16_t* vt_img;               // 2 x [Hkv][tiles][128][64]
+  int* vexp;                      // [Hkv][tiles] exponents of the V tiles
+  int* vmax;                      // [layers] largest of them
+  unsigned* argmax_count;         // [64] cleared for the lm_head
+};
+struct PrefillPlan {
+  GemmPlan qkv, o_proj, gate_up, down;
+  long part_floats;
+};
+PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I);
+// Every layer; leaves the last row of the residual stream in h.
+int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const PrefillPlan& p, hipStream_t s);
+
 }  // namespace qd

@@ -1,0 +1,847 @@
+// Prompt prefill for gfx950: the decoder layers over S prompt rows with fp32
+// arithmetic carried on the fp16 matrix cores, the K/V rows written to the
+// static cache, and the last row's greedy token.
+//
+// fp32 on fp16 MFMA.  The weights are fp16, so only the activations need more
+// than one fp16 value: an activation row x is scaled by a power of two that
+// puts its largest value in [2^13, 2^14) and split into hi = fp16(x) and
+// lo = fp16(x - hi), 22 bits in all (values down to 2^-15 of the largest keep
+// them; below that the split's absolute error is 2^-39 of the largest).
+// W.x = W.hi + W.lo then takes two MFMAs per tile with exact products and
+// fp32 accumulation.  Measured against 64 bits on N(0, 1) rows, K = 2048: 4.1e-7
+// relative, where an fp32 GEMM has 8.1e-7.  gfx950 has no faster fp32-input
+// MFMA (157 TFLOP/s, against 2 x 16 bits of 2500).
+//
+// One layer is nine launches:
+//   rows      h += the previous GEMM's partials; RMSNorm; split image + scale
+//   gemm      qkv partials
+//   qkv_prep  q/k head RMSNorm + M-RoPE, K/V cache rows, split images of q, k
+//             and of V transposed (the attention's operand orders)
+//   attention causal flash attention on the split images, split image out
+//   gemm      o_proj partials
+//   rows      h += partials; RMSNorm; split image
+//   gemm      gate_up partials
+//   silu      silu(gate) * up, split image + scale
+//   gemm      down partials
+// A GEMM may split K over z workgroups per tile (few rows, where a tile grid
+// leaves CUs idle); its z partial planes are summed in order by the next
+// launch, which reads them anyway.
+//
+// Replaces the prefill of the reference's greedy engine
+// (evaluation_wrapper.py:218-228, a full HF forward).
+
+#include <math.h>
+
+#include <type_traits>
+
+#include "qd_common.h"
+#include "qd_kernels.h"
+
+namespace qd {
+
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+constexpr int kHD = 128;        // head dim
+constexpr int kKvTile = 64;     // K/V rows per attention tile
+constexpr int kMaxExp = 110;
+
+// ---------------------------------------------------------------- fp16 splits
+
+// Exponent e with amax * 2^-e in [2^13, 2^14), clamped so that 2^e and 2^-e
+// are normal fp32 numbers (0 and non-finite maxima give a clamped one).
+__device__ __forceinline__ int split_exp(float amax) {
+  const int e = (int)((__builtin_bit_cast(unsigned, amax) >> 23) & 0xffu) - 127 - 13;
+  return min(max(e, -kMaxExp), kMaxExp);
+}
+__device__ __forceinline__ float pow2f(int e) {   // -126 <= e <= 127
+  return __builtin_bit_cast(float, (unsigned)(e + 127) << 23);
+}
+// x is made opaque first: where it is a product, the compiler may otherwise
+// round the stored hi straight from the exact product (v_fma_mixlo_f16) and the
+// hi inside lo from the fp32 product, which differ by an fp16 step now and then.
+__device__ __forceinline__ void split2(float x, _Float16& hi, _Float16& lo) {
+  asm("" : "+v"(x));
+  hi = (_Float16)x;
+  lo = (_Float16)(x - (float)hi);
+}
+
+// 8 consecutive values (already scaled) to the two planes.
+__device__ __forceinline__ void store_split8(uint16_t* hi, uint16_t* lo, const float* u) {
+  h8 a, b;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    _Float16 x, y;
+    split2(u[i], x, y);
+    a[i] = x;
+    b[i] = y;
+  }
+  *reinterpret_cast<h8*>(hi) = a;
+  *reinterpret_cast<h8*>(lo) = b;
+}
+
+__device__ __forceinline__ float block_max(float v, float* s_red, int nw) {
+  v = wave_max(v);
+  if (lane_id() == 0) s_red[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = s_red[0];
+  for (int i = 1; i < nw; ++i) v = fmaxf(v, s_red[i]);
+  __syncthreads();
+  return v;
+}
+__device__ __forceinline__ float block_sum(float v, float* s_red, int nw) {
+  v = wave_sum(v);
+  if (lane_id() == 0) s_red[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = s_red[0];
+  for (int i = 1; i < nw; ++i) v += s_red[i];
+  __syncthreads();
+  return v;
+}
+
+// ---------------------------------------------------------------- asynchronous LDS tiles
+
+// A word at a wave-uniform address, written by an earlier launch, as a scalar
+// load: a vector load would make its reader wait for the tile loads in flight.
+__device__ __forceinline__ int ld_scalar(const int* p) {
+  return *(const __attribute__((address_space(4))) int*)p;
+}
+
+// 16 bytes per lane from global memory straight to LDS (lane i lands at
+// l + 16 i; l is wave-uniform).
+__device__ __forceinline__ void load_lds16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                   (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+
+// This wave's LDS reads are done and at most N of its loads are in flight,
+// then the workgroup barrier.  The loads that a tile's readers need are older
+// than the N allowed ones, and a tile is refilled only after the barrier that
+// follows its last read.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0070);   // vmcnt(N) lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+// Stage I of a kernel's tile ring.  Separate variables, not slices of one: the
+// compiler then knows that reading one stage does not depend on the loads in
+// flight to another and puts no wait of its own between them.
+template <int I, int N>
+__device__ __forceinline__ char* lds_stage() {
+  __shared__ __align__(16) char buf[N];
+  return buf;
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------- split GEMM
+
+// y[z][m][n] = scale[m] * sum over the z-th K range of W[n][k] (hi + lo)[m][k].
+//
+// Tile BM x BN, BK of K per stage (hi, lo and W rows), NS stages filled by
+// asynchronous global-to-LDS loads NS - 1 steps ahead.  16-byte chunk c of row
+// r sits at c ^ (r % 8) (rows of 128 bytes; c ^ (r / 2 % 4) for 64), so that
+// the 16 rows a fragment read touches spread over all banks; the permutation is
+// applied to the source address, since the load's LDS side is contiguous.  W is
+// the MFMA A operand, so a lane holds four consecutive outputs of one row.
+// Consecutive tiles of one XCD share their W rows (the m tiles of one n band),
+// which then come out of its L2.
+template <int BM, int BN, int BK, int WM, int WN, int NS>
+__global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const SplitGemmArgs a) {
+  constexpr int NW = WM * WN;
+  constexpr int TM = BM / WM, TN = BN / WN;
+  constexpr int CH = BK / 8;
+  constexpr int RPI = kWave / CH;                       // rows per load
+  constexpr int LA = BM / RPI / NW, LW = BN / RPI / NW;  // loads per wave and stage
+  constexpr int LOADS = 2 * LA + LW;
+  constexpr int PA = 2 * BM * BK, STAGE = 2 * PA + 2 * BN * BK;   // bytes
+  static_assert(LA >= 1 && LW >= 1 && (CH == 8 || CH == 4) && LOADS * (NS - 1) < 64 && NS == 3, "tile shape");
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int tiles_m = (a.M + BM - 1) / BM;
+  const int q = (int)gridDim.x >> 3, r = (int)gridDim.x & 7, xcd = (int)blockIdx.x & 7, loc = (int)blockIdx.x >> 3;
+  const int t = xcd * q + min(xcd, r) + loc;
+  const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
+  const int kz = a.K / (int)gridDim.y, nk = kz / BK;
+  const long kbase = (long)blockIdx.y * kz;
+  const int lr = lane / CH, lc = lane % CH;
+  const int sc = lc ^ (CH == 8 ? (lr & 7) : ((lr >> 1) & 3));
+  unsigned offA[LA], offW[LW];
+#pragma unroll
+  for (int i = 0; i < LA; ++i)
+    offA[i] = ((unsigned)min(m0 + (i * NW + w) * RPI + lr, a.M - 1) * (unsigned)a.K + sc * 8) * 2u;
+#pragma unroll
+  for (int i = 0; i < LW; ++i)
+    offW[i] = ((unsigned)min(n0 + (i * NW + w) * RPI + lr, a.N - 1) * (unsigned)a.K + sc * 8) * 2u;
+  const char* Ah = reinterpret_cast<const char*>(a.hi + kbase);
+  const char* Al = reinterpret_cast<const char*>(a.lo + kbase);
+  const char* Wp = reinterpret_cast<const char*>(a.W + kbase);
+  auto issue = [&](auto S, int k) {
+    char* st = lds_stage<decltype(S)::value, STAGE>();
+    const long ko = (long)k * BK * 2;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      load_lds16(Ah + ko + offA[i], st + (i * NW + w) * 1024);
+      load_lds16(Al + ko + offA[i], st + PA + (i * NW + w) * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < LW; ++i) load_lds16(Wp + ko + offW[i], st + 2 * PA + (i * NW + w) * 1024);
+  };
+  f32x4 acc[TM / 16][TN / 16];
+#pragma unroll
+  for (int i = 0; i < TM / 16; ++i)
+#pragma unroll
+    for (int j = 0; j < TN / 16; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = w / WN, wn = w % WN;
+  const int fr = lane & 15, fg = lane >> 4;
+  const int fs = CH == 8 ? (fr & 7) : ((fr >> 1) & 3);
+  // byte offsets of this lane's fragments, opaque so that every fragment
+  // address stays one base plus a constant
+  unsigned bA[BK / 32], bW[BK / 32];
+#pragma unroll
+  for (int ks = 0; ks < BK / 32; ++ks) {
+    const unsigned co = ((4 * ks + fg) ^ fs) * 16;
+    bA[ks] = (wm * TM + fr) * BK * 2 + co;
+    bW[ks] = 2 * PA + (wn * TN + fr) * BK * 2 + co;
+    asm("" : "+v"(bA[ks]));
+    asm("" : "+v"(bW[ks]));
+  }
+  auto compute = [&](auto S) {
+    const char* st = lds_stage<decltype(S)::value, STAGE>();
+#pragma unroll
+    for (int ks = 0; ks < BK / 32; ++ks) {
+      h8 fw[TN / 16];
+#pragma unroll
+      for (int j = 0; j < TN / 16; ++j) fw[j] = *reinterpret_cast<const h8*>(st + bW[ks] + 32 * j * BK);
+#pragma unroll
+      for (int i = 0; i < TM / 16; ++i) {
+        const h8 fh = *reinterpret_cast<const h8*>(st + bA[ks] + 32 * i * BK);
+        const h8 fl = *reinterpret_cast<const h8*>(st + bA[ks] + PA + 32 * i * BK);
+#pragma unroll
+        for (int j = 0; j < TN / 16; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fh, acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < TN / 16; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j], fl, acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  auto full = [&](auto S, int k) {   // steady state: stage k + 2 is refilled while k is used
+    wait_barrier<LOADS>();
+    issue(std::integral_constant<int, (decltype(S)::value + 2) % 3>{}, k + 2);
+    compute(S);
+  };
+  auto tail = [&](auto S, int k) {
+    if (k >= nk) return;
+    if (k + 1 < nk)
+      wait_barrier<LOADS>();
+    else
+      wait_barrier<0>();
+    if (k + 2 < nk) issue(std::integral_constant<int, (decltype(S)::value + 2) % 3>{}, k + 2);
+    compute(S);
+  };
+  const std::integral_constant<int, 0> s0;
+  const std::integral_constant<int, 1> s1;
+  const std::integral_constant<int, 2> s2;
+  issue(s0, 0);
+  if (nk > 1) issue(s1, 1);
+  int k = 0;
+#pragma unroll 1
+  for (; k + 4 < nk; k += 3) {
+    full(s0, k);
+    full(s1, k + 1);
+    full(s2, k + 2);
+  }
+#pragma unroll 1
+  for (; k < nk; k += 3) {
+    tail(s0, k);
+    tail(s1, k + 1);
+    tail(s2, k + 2);
+  }
+  float scale[TM / 16];
+#pragma unroll
+  for (int i = 0; i < TM / 16; ++i)
+    scale[i] = a.scale[(long)min(m0 + wm * TM + 16 * i + fr, a.M - 1) * a.scale_stride];
+  float* y = a.y + (long)blockIdx.y * a.M * a.N;
+#pragma unroll
+  for (int i = 0; i < TM / 16; ++i) {
+    const int m = m0 + wm * TM + 16 * i + fr;
+    if (m < a.M) {
+#pragma unroll
+      for (int j = 0; j < TN / 16; ++j) {
+        const int n = n0 + wn * TN + 16 * j + 4 * fg;
+        if (n < a.N) *reinterpret_cast<f32x4*>(y + (long)m * a.N + n) = acc[i][j] * scale[i];
+      }
+    }
+  }
+}
+
+namespace {
+
+// Tile shapes and their cost: a workgroup's microseconds per 1024 of K with
+// every CU busy (measured, S = 1024 and 4001 at the 2B shapes) and how many
+// share a CU.
+struct GemmTile {
+  int bm, bn, bk, per_cu;
+  float us;
+};
+constexpr GemmTile kGemmTiles[] = {
+    {256, 256, 32, 1, 57.f},   // 1144 TFLOP/s of MFMA at 4001 x 12288 x 2048
+    {128, 128, 64, 1, 20.f},   // 824 at 1024 x 4096 x 2048
+    {64, 128, 64, 1, 13.f},
+    {64, 64, 64, 2, 13.f},
+};
+
+template <int BM, int BN, int BK, int WM, int WN>
+int launch_gemm(const SplitGemmArgs& a, int z, hipStream_t s) {
+  const unsigned t = (unsigned)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
+  hipLaunchKernelGGL((split_gemm_kernel<BM, BN, BK, WM, WN, 3>), dim3(t, (unsigned)z), dim3(kWave * WM * WN), 0, s, a);
+  return qd_host::launch_status("split_gemm_kernel");
+}
+
+}  // namespace
+
+// The tile shape and K split with the least estimated time: rounds of
+// workgroups over the CUs, each costing its K range's tile time plus a fixed
+// ~3 us, plus the partial planes written and read again (~4 TB/s).
+GemmPlan split_gemm_plan(long M, long N, long K) {
+  GemmPlan best{-1, 1};
+  float best_us = 0.f;
+  const int cus = qd_host::cu_count();
+  for (int c = 0; c < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++c) {
+    const GemmTile& g = kGemmTiles[c];
+    for (int z = 1; z <= kPrefillMaxSplit; z *= 2) {
+      if (K % ((long)g.bk * z) != 0) break;
+      const long wgs = ((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn) * z;
+      const long rounds = (wgs + (long)cus * g.per_cu - 1) / ((long)cus * g.per_cu);
+      const float us = (float)rounds * (3.f + g.us * (float)(K / z) / 1024.f) +
+                       8.f * (float)z * (float)M * (float)N / 4e6f;
+      if (best.tile < 0 || us < best_us) {
+        best = GemmPlan{c, z};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+int split_gemm_launch(const SplitGemmArgs& a, const GemmPlan& p, hipStream_t s) {
+  if (a.M < 1 || a.N < 4 || a.N % 4 != 0 || p.tile < 0 || p.z < 1 || a.K % ((long)kGemmTiles[p.tile].bk * p.z) != 0)
+    return QD_ERR_SHAPE;
+  // 32-bit byte offsets into the operands
+  if ((size_t)a.M * a.K * 2 >> 32 || (size_t)a.N * a.K * 2 >> 32) return QD_ERR_SHAPE;
+  switch (p.tile) {
+    case 0: return launch_gemm<256, 256, 32, 2, 4>(a, p.z, s);
+    case 1: return launch_gemm<128, 128, 64, 2, 2>(a, p.z, s);
+    case 2: return launch_gemm<64, 128, 64, 2, 2>(a, p.z, s);
+    default: return launch_gemm<64, 64, 64, 2, 2>(a, p.z, s);
+  }
+}
+
+namespace {
+
+// ---------------------------------------------------------------- elementwise launches
+
+// cos / sin of every (row, rotary pair), fp32 angles as the decode step's, and
+// the words that must start at zero (exponent maxima, the argmax counter).
+__global__ __launch_bounds__(256) void prefill_init_kernel(const PrefillArgs a) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < a.layers_n) a.vmax[i] = -kMaxExp;
+  if (i < 64) a.argmax_count[i] = 0u;
+  if (i >= (long)a.S * (kHD / 2)) return;
+  const int row = (int)(i / (kHD / 2)), j = (int)(i % (kHD / 2));
+  int st = 0;
+  if (j % 3 == 1 && j < 3 * a.sec_h) st = 1;
+  if (j % 3 == 2 && j < 3 * a.sec_w) st = 2;
+  float s, c;
+  sincosf((float)a.position_ids[(long)st * a.S + row] * a.inv_freq[j], &s, &c);
+  a.cs[i] = make_float2(c, s);
+}
+
+constexpr int kRowChunks = 4;   // 8-value chunks per thread of a row: H up to 8192
+
+// One row per workgroup: h[row] (+ the GEMM's z partial rows, or the prompt's
+// embedding instead, layer 0), RMSNorm, split image and its scale.  HBM / L2
+// bound: reads (z + 1) and writes 2 x 4 bytes per value.
+template <bool EMBED>
+__global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, const float* part, int z,
+                                                           const uint16_t* gamma, int row0) {
+  __shared__ float s_red[4];
+  const int row = row0 + (int)blockIdx.x;
+  const long H = a.H;
+  float* hr = a.h + row * H;
+  float u[kRowChunks][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < kRowChunks; ++c) {
+    const long k = (long)c * 2048 + threadIdx.x * 8;
+    if (k >= H) continue;
+    if constexpr (EMBED) {
+      if (row < a.n_vision) {
+        if (a.vision_f32)
+          load_act8<float>(reinterpret_cast<const float*>(a.vision) + row * H, k, u[c]);
+        else
+          load_act8<uint16_t>(reinterpret_cast<const uint16_t*>(a.vision) + row * H, k, u[c]);
+      } else {
+        load_act8<uint16_t>(a.embed + a.text_ids[row - a.n_vision] * H, k, u[c]);
+      }
+    } else {
+      load_act8<float>(hr, k, u[c]);
+      float p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < z; ++i) {
+        float v[8];
+        load_act8<float>(part + ((long)i * a.S + row) * H, k, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] += v[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) u[c][e] += p[e];
+    }
+    store_act8<float>(hr, k, u[c]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(u[c][e], u[c][e], ss);
+  }
+  if (gamma == nullptr) return;   // after the last layer only h is wanted
+  const float rstd = rsqrtf(block_sum(ss, s_red, 4) / (float)H + a.eps);
+  float mx = 0.f;
+#pragma unroll
+  for (int c = 0; c < kRowChunks; ++c) {
+    const long k = (long)c * 2048 + threadIdx.x * 8;
+    if (k >= H) continue;
+    float g[8];
+    unpack8(ld16(gamma + k), g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      u[c][e] = (u[c][e] * rstd) * g[e];
+      mx = fmaxf(mx, fabsf(u[c][e]));
+    }
+  }
+  const int e2 = split_exp(block_max(mx, s_red, 4));
+  const float sc = pow2f(-e2);
+#pragma unroll
+  for (int c = 0; c < kRowChunks; ++c) {
+    const long k = (long)c * 2048 + threadIdx.x * 8;
+    if (k >= H) continue;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) u[c][e] *= sc;
+    store_split8(a.img + row * H + k, a.img + ((long)a.S + row) * H + k, u[c]);
+  }
+  if (threadIdx.x == 0) a.scale[row] = pow2f(e2);
+}
+
+constexpr int kSiluChunks = 8;   // I up to 16384
+
+// One row per workgroup: hidden = silu(gate) * up from the gate_up partials,
+// split image and scale.
+__global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, int z) {
+  __shared__ float s_red[4];
+  const int row = blockIdx.x;
+  const long I = a.I;
+  float u[kSiluChunks][8];
+  float mx = 0.f;
+#pragma unroll
+  for (int c = 0; c < kSiluChunks; ++c) {
+    const long k = (long)c * 2048 + threadIdx.x * 8;
+    if (k >= I) continue;
+    float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < z; ++i) {
+      const float* src = a.part + ((long)i * a.S + row) * 2 * I;
+      float v[8], w[8];
+      load_act8<float>(src, k, v);
+      load_act8<float>(src + I, k, w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        g[e] += v[e];
+        p[e] += w[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      u[c][e] = (g[e] / (1.0f + expf(-g[e]))) * p[e];
+      mx = fmaxf(mx, fabsf(u[c][e]));
+    }
+  }
+  const int e2 = split_exp(block_max(mx, s_red, 4));
+  const float sc = pow2f(-e2);
+#pragma unroll
+  for (int c = 0; c < kSiluChunks; ++c) {
+    const long k = (long)c * 2048 + threadIdx.x * 8;
+    if (k >= I) continue;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) u[c][e] *= sc;
+    store_split8(a.img + row * I + k, a.img + ((long)a.S + row) * I + k, u[c]);
+  }
+  if (threadIdx.x == 0) a.scale[row] = pow2f(e2);
+}
+
+// Exponent of a head-normalised and rotated vector's image: |x| <= sqrt(2 D) max |w|.
+__device__ __forceinline__ int head_exp(const uint16_t* w) {
+  const int j = lane_id();
+  const float m = wave_max(fmaxf(fabsf(h2f(w[j])), fabsf(h2f(w[j + kHD / 2]))));
+  return split_exp(m * 16.f);
+}
+
+// Workgroups [0, q/k groups): one wave per (row, q or k head): head RMSNorm,
+// rotation, split image; k also to the cache.  The others: one (kv head, 64
+// rows) tile of V each: cache rows, and the split image of the tile transposed,
+// [128 dims][64 rows] with the rows of each half in the order the PV product's
+// operand holds its probabilities in: position 8 g + e is row
+// 16 (e / 4) + 4 g + e % 4.  The tile's exponent goes to vexp and, as the layer's
+// maximum, to vmax.
+__global__ __launch_bounds__(256) void prefill_qkv_prep_kernel(const PrefillArgs a, const PrefillLayer L, int z,
+                                                               int qk_groups, int layer) {
+  __shared__ float s_red[4];
+  const long NQ = (long)(a.Hq + 2 * a.Hkv) * kHD;
+  if ((int)blockIdx.x < qk_groups) {
+    const long item = (long)blockIdx.x * 4 + threadIdx.x / kWave;
+    const int heads = a.Hq + a.Hkv;
+    const int row = (int)(item / heads), head = (int)(item % heads);
+    if (row >= a.S) return;
+    const int j = lane_id();
+    const bool is_q = head < a.Hq;
+    float x0 = 0.f, x1 = 0.f;
+    for (int i = 0; i < z; ++i) {
+      const float* src = a.part + ((long)i * a.S + row) * NQ + (long)head * kHD;
+      x0 += src[j];
+      x1 += src[j + kHD / 2];
+    }
+    const uint16_t* nw = is_q ? L.q_norm : L.k_norm;
+    const float2 cs = a.cs[(long)row * (kHD / 2) + j];
+    const float rstd = rsqrtf(wave_sum(x0 * x0 + x1 * x1) / (float)kHD + a.eps);
+    const float n0 = (x0 * rstd) * h2f(nw[j]), n1 = (x1 * rstd) * h2f(nw[j + kHD / 2]);
+    const float o0 = n0 * cs.x - n1 * cs.y, o1 = n1 * cs.x + n0 * cs.y;
+    const int e = head_exp(nw);
+    const float sc = pow2f(-e);
+    _Float16 h0, l0, h1, l1;
+    split2(o0 * sc, h0, l0);
+    split2(o1 * sc, h1, l1);
+    const int hh = is_q ? head : head - a.Hq;
+    const long plane = (long)(is_q ? a.Hq : a.Hkv) * a.S * kHD;
+    _Float16* dst = reinterpret_cast<_Float16*>(is_q ? a.q_img : a.k_img) + ((long)hh * a.S + row) * kHD;
+    dst[j] = h0;
+    dst[j + kHD / 2] = h1;
+    dst[plane + j] = l0;
+    dst[plane + j + kHD / 2] = l1;
+    if (!is_q) {
+      uint16_t* kc = L.k_cache + ((long)hh * a.T + row) * kHD;
+      kc[j] = f2h(o0);
+      kc[j + kHD / 2] = f2h(o1);
+    }
+    return;
+  }
+  const int tiles = (a.S + kKvTile - 1) / kKvTile;
+  const int it = (int)blockIdx.x - qk_groups;
+  const int kvh = it / tiles, tile = it % tiles;
+  const int d = threadIdx.x & (kHD - 1), half = threadIdx.x / kHD;
+  const int r0 = tile * kKvTile + half * 32;
+  float v[32];
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    v[i] = 0.f;
+    if (r0 + i < a.S) {
+      for (int p = 0; p < z; ++p)
+        v[i] += a.part[((long)p * a.S + r0 + i) * NQ + (long)(a.Hq + a.Hkv + kvh) * kHD + d];
+      L.v_cache[((long)kvh * a.T + r0 + i) * kHD + d] = f2h(v[i]);
+      mx = fmaxf(mx, fabsf(v[i]));
+    }
+  }
+  const int e = split_exp(block_max(mx, s_red, 4));
+  const float sc = pow2f(-e);
+  const long plane = (long)a.Hkv * tiles * kHD * kKvTile;
+  uint16_t* dst = a.vt_img + ((long)it * kHD + d) * kKvTile + half * 32;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    float u[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) u[x] = v[16 * (x / 4) + 4 * g + x % 4] * sc;
+    store_split8(dst + 8 * g, dst + plane + 8 * g, u);
+  }
+  if (threadIdx.x == 0) {
+    a.vexp[it] = e;
+    atomicMax(a.vmax + layer, e);
+  }
+}
+
+// ---------------------------------------------------------------- causal attention
+
+// One workgroup: one q head, 4 waves of 16 QT rows each, the K/V tiles of 64
+// rows up to the diagonal.  S^T = K.Q^T and O^T = V^T.P^T, so that a lane's
+// probabilities (one q row, 4 + 4 kv rows per 32) already are the operand of
+// the second product, and the softmax's row factors are one value per lane.  Each
+// product of split operands is three MFMAs (hi.hi + lo.hi + hi.lo; the dropped
+// lo.lo is 2^-22 of a term).  Probabilities are scaled by 2^13 and by the V
+// tile's exponent against the layer's largest, which keeps them in fp16 range
+// and the accumulators in one unit, 2^(vmax - 13); the output's split image
+// takes 2^vmax as its scale (|o| <= the layer's largest |v|).
+//
+// K and V tiles (32 KB each) are single-buffered: the next K tile is requested
+// when the scores are done, the next V tile after the second product, and two
+// workgroups share a CU, each computing while the other waits.
+template <int QT>
+__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L, int layer,
+                                                                   int q_tiles) {
+  constexpr int kPlane = kKvTile * kHD * 2;   // bytes of one K or V plane of a tile
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int c = lane & 15, g = lane >> 4;
+  // heavy (late) tiles first; one kv head's workgroups share an XCD's L2 when Hkv = 8
+  const int kvh = (int)blockIdx.x % a.Hkv, rest = (int)blockIdx.x / a.Hkv;
+  const int group = a.Hq / a.Hkv;
+  const int head = kvh * group + rest % group;
+  const int qt = q_tiles - 1 - rest / group;
+  const int q0 = qt * 64 * QT + w * 16 * QT;    // this wave's first row
+  const int tiles = (a.S + kKvTile - 1) / kKvTile;
+  const int nt = min((qt + 1) * QT, tiles);
+  const long kplane = (long)a.Hkv * a.S * kHD, vplane = (long)a.Hkv * tiles * kHD * kKvTile;
+  const uint16_t* ki = a.k_img + (long)kvh * a.S * kHD;
+  const uint16_t* vi = a.vt_img + (long)kvh * tiles * kHD * kKvTile;
+
+  // K tile: 64 rows of 16 chunks, 4 rows per load, chunk c of row r at
+  // c ^ (r % 8); V tile: 128 rows (dims) of 8 chunks, 8 rows per load.  Wave w
+  // loads rows [16 w, 16 w + 16) of both K planes and dims [32 w, 32 w + 32) of V.
+  auto issue_k = [&](int t) {
+    char* st = lds_stage<0, 2 * kPlane>();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * w + 4 * i + (lane >> 4);
+      const int ch = (lane & 15) ^ (r & 7);
+      const uint16_t* src = ki + (long)min(t * kKvTile + r, a.S - 1) * kHD + ch * 8;
+      load_lds16(src, st + (16 * w + 4 * i) * 256);
+      load_lds16(src + kplane, st + kPlane + (16 * w + 4 * i) * 256);
+    }
+  };
+  auto issue_v = [&](int t) {
+    char* st = lds_stage<1, 2 * kPlane>();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 32 * w + 8 * i + (lane >> 3);
+      const int ch = (lane & 7) ^ (r & 7);
+      const uint16_t* src = vi + ((long)t * kHD + r) * kKvTile + ch * 8;
+      load_lds16(src, st + (32 * w + 8 * i) * 128);
+      load_lds16(src + vplane, st + kPlane + (32 * w + 8 * i) * 128);
+    }
+  };
+  issue_k(0);
+  issue_v(0);
+
+  // Q operand: column c = row q0 + 16 i + c, k 8 g .. 8 g + 7 of each 32 dims
+  h8 qh[QT][4], ql[QT][4];
+  const long qplane = (long)a.Hq * a.S * kHD;
+#pragma unroll
+  for (int i = 0; i < QT; ++i) {
+    const uint16_t* src = a.q_img + ((long)head * a.S + min(q0 + 16 * i + c, a.S - 1)) * kHD + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      qh[i][ks] = *reinterpret_cast<const h8*>(src + 32 * ks);
+      ql[i][ks] = *reinterpret_cast<const h8*>(src + qplane + 32 * ks);
+    }
+  }
+  const int emax = a.vmax[layer];
+  // log2 units: scale * log2(e) * 2^(q exponent + k exponent)
+  const float fac = a.attn_scale * 1.44269504088896340736f * pow2f(head_exp(L.q_norm)) * pow2f(head_exp(L.k_norm));
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.o_scale[0] = pow2f(emax);
+
+  f32x4 o[QT][8];
+  float m[QT], l[QT];
+#pragma unroll
+  for (int i = 0; i < QT; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  unsigned bk[4], bv[2];   // this lane's fragment bases (opaque, see split_gemm_kernel)
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    bk[ks] = c * 256 + (((4 * ks + g) ^ (c & 7)) << 4);
+    asm("" : "+v"(bk[ks]));
+  }
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    bv[ks] = c * 128 + (((4 * ks + g) ^ (c & 7)) << 4);
+    asm("" : "+v"(bv[ks]));
+  }
+
+#pragma unroll 1
+  for (int t = 0; t < nt; ++t) {
+    wait_barrier<8>();   // K tile t (V tile t may be in flight)
+    const int ve = ld_scalar(a.vexp + kvh * tiles + t);
+    const char* sk = lds_stage<0, 2 * kPlane>();
+    f32x4 s[QT][4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+      for (int i = 0; i < QT; ++i) s[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const h8 kh = *reinterpret_cast<const h8*>(sk + bk[ks] + n * 16 * 256);
+        const h8 kl = *reinterpret_cast<const h8*>(sk + bk[ks] + kPlane + n * 16 * 256);
+#pragma unroll
+        for (int i = 0; i < QT; ++i) {
+          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[i][ks], s[i][n], 0, 0, 0);
+          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[i][ks], s[i][n], 0, 0, 0);
+          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[i][ks], s[i][n], 0, 0, 0);
+        }
+      }
+    }
+    wait_barrier<8>();   // every wave is done with K tile t (this wave's V loads stay in flight)
+    issue_k(min(t + 1, nt - 1));
+
+    const float cv = ve - emax + 13 > -126 ? pow2f(ve - emax + 13) : 0.f;
+    const bool diag = t * kKvTile + kKvTile - 1 > q0;
+    h8 ph[QT][2], pl[QT][2];
+#pragma unroll
+    for (int i = 0; i < QT; ++i) {
+      const int lim = q0 + 16 * i + c - t * kKvTile - 4 * g;   // kv 16 n + 4 g + j is visible up to lim
+      float mx = -INFINITY;
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float v = s[i][n][j] * fac;
+          if (diag && 16 * n + j > lim) v = -INFINITY;
+          s[i][n][j] = v;
+          mx = fmaxf(mx, v);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = fmaxf(m[i], mx);
+      const float al = __builtin_amdgcn_exp2f(m[i] - mn);
+      m[i] = mn;
+      float ps = 0.f;
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p = __builtin_amdgcn_exp2f(s[i][n][j] - mn);
+          ps += p;
+          _Float16 hi, lo;
+          split2(p * cv, hi, lo);
+          ph[i][n / 2][4 * (n & 1) + j] = hi;
+          pl[i][n / 2][4 * (n & 1) + j] = lo;
+        }
+      l[i] = __builtin_fmaf(l[i], al, ps);
+#pragma unroll
+      for (int d = 0; d < 8; ++d) o[i][d] *= al;
+    }
+    wait_barrier<8>();   // V tile t (K tile t + 1 may be in flight)
+    const char* sv = lds_stage<1, 2 * kPlane>();
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const h8 vh = *reinterpret_cast<const h8*>(sv + bv[ks] + d * 16 * 128);
+        const h8 vl = *reinterpret_cast<const h8*>(sv + bv[ks] + kPlane + d * 16 * 128);
+#pragma unroll
+        for (int i = 0; i < QT; ++i) {
+          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[i][ks], o[i][d], 0, 0, 0);
+          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[i][ks], o[i][d], 0, 0, 0);
+          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[i][ks], o[i][d], 0, 0, 0);
+        }
+      }
+    wait_barrier<8>();   // every wave is done with V tile t
+    issue_v(min(t + 1, nt - 1));
+  }
+  const long HD = (long)a.Hq * kHD;
+#pragma unroll
+  for (int i = 0; i < QT; ++i) {
+    l[i] += __shfl_xor(l[i], 16);
+    l[i] += __shfl_xor(l[i], 32);
+    const int row = q0 + 16 * i + c;
+    const float inv = 1.f / (8192.f * l[i]);
+    if (row < a.S) {
+      uint16_t* dst = a.img + (long)row * HD + (long)head * kHD + 4 * g;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        h4 hi, lo;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          _Float16 x, y;
+          split2(o[i][d][j] * inv, x, y);
+          hi[j] = x;
+          lo[j] = y;
+        }
+        *reinterpret_cast<h4*>(dst + 16 * d) = hi;
+        *reinterpret_cast<h4*>(dst + (long)a.S * HD + 16 * d) = lo;
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);   // the last (unused) tiles have landed before the LDS is given back
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------- host
+
+PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I) {
+  PrefillPlan p;
+  const long qn = (long)(Hq + 2 * Hkv) * kHD, qs = (long)Hq * kHD;
+  p.qkv = split_gemm_plan(S, qn, H);
+  p.o_proj = split_gemm_plan(S, H, qs);
+  p.gate_up = split_gemm_plan(S, 2L * I, H);
+  p.down = split_gemm_plan(S, H, I);
+  const long n[4] = {p.qkv.z * qn, (long)p.o_proj.z * H, p.gate_up.z * 2L * I, (long)p.down.z * H};
+  p.part_floats = 0;
+  for (long x : n)
+    if (x * S > p.part_floats) p.part_floats = x * S;
+  return p;
+}
+
+int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const PrefillPlan& p, hipStream_t s) {
+  const int tiles = (a.S + kKvTile - 1) / kKvTile;
+  const int qs = a.Hq * kHD, qn = (a.Hq + 2 * a.Hkv) * kHD;
+  int st;
+  const long rot = (long)a.S * (kHD / 2), init = rot > a.layers_n ? rot : a.layers_n;
+  hipLaunchKernelGGL(prefill_init_kernel, dim3((unsigned)((init + 255) / 256)), dim3(256), 0, s, a);
+  if ((st = qd_host::launch_status("prefill_init_kernel"))) return st;
+  auto gemm = [&](const uint16_t* W, const float* scale, int scale_stride, int N, int K, const GemmPlan& g) {
+    SplitGemmArgs x;
+    x.hi = a.img; x.lo = a.img + (long)a.S * K; x.scale = scale; x.scale_stride = scale_stride; x.W = W; x.y = a.part;
+    x.M = a.S; x.N = N; x.K = K;
+    return split_gemm_launch(x, g, s);
+  };
+  const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + 3) / 4);
+  // 128 q rows per workgroup once that still gives every CU two workgroups
+  const bool wide = (long)((a.S + 127) / 128) * a.Hq >= 2L * qd_host::cu_count();
+  const int q_tiles = wide ? (a.S + 127) / 128 : (a.S + 63) / 64;
+  for (int li = 0; li < a.layers_n; ++li) {
+    const PrefillLayer& L = layers[li];
+    if (li == 0)
+      hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((unsigned)a.S), dim3(256), 0, s, a, nullptr, 0, L.input_norm, 0);
+    else
+      hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((unsigned)a.S), dim3(256), 0, s, a, a.part, p.down.z,
+                         L.input_norm, 0);
+    if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
+    if ((st = gemm(L.qkv, a.scale, 1, qn, a.H, p.qkv))) return st;
+    hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)), dim3(256), 0, s, a, L,
+                       p.qkv.z, qk_groups, li);
+    if ((st = qd_host::launch_status("prefill_qkv_prep_kernel"))) return st;
+    if (wide)
+      hipLaunchKernelGGL((prefill_attention_kernel<2>), dim3((unsigned)(q_tiles * a.Hq)), dim3(256), 0, s, a, L, li,
+                         q_tiles);
+    else
+      hipLaunchKernelGGL((prefill_attention_kernel<1>), dim3((unsigned)(q_tiles * a.Hq)), dim3(256), 0, s, a, L, li,
+                         q_tiles);
+    if ((st = qd_host::launch_status("prefill_attention_kernel"))) return st;
+    if ((st = gemm(L.o_proj, a.o_scale, 0, a.H, qs, p.o_proj))) return st;
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((unsigned)a.S), dim3(256), 0, s, a, a.part, p.o_proj.z,
+                       L.post_norm, 0);
+    if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
+    if ((st = gemm(L.gate_up, a.scale, 1, 2 * a.I, a.H, p.gate_up))) return st;
+    hipLaunchKernelGGL(prefill_silu_kernel, dim3((unsigned)a.S), dim3(256), 0, s, a, p.gate_up.z);
+    if ((st = qd_host::launch_status("prefill_silu_kernel"))) return st;
+    if ((st = gemm(L.down, a.scale, 1, a.H, a.I, p.down))) return st;
+  }
+  hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3(1), dim3(256), 0, s, a, a.part, p.down.z, nullptr, a.S - 1);
+  return qd_host::launch_status("prefill_rows_kernel");
+}
+
+}  // namespace qd

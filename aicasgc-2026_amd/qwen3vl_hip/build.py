@@ -20,7 +20,8 @@ CSRC = PKG_ROOT / "csrc"
 LIB_NAME = "libqwen3vl_decode.so"
 LIB_PATH = PKG_ROOT / LIB_NAME
 TRACE_LIB_PATH = PKG_ROOT / "libqwen3vl_decode_trace.so"   # same sources with -DQD_TRACE
-SOURCES = ["qd_gemv.hip", "qd_attention.hip", "qd_small_ops.hip", "qd_persistent.hip", "qd_batch.hip", "qd_capi.hip"]
+SOURCES = ["qd_gemv.hip", "qd_attention.hip", "qd_small_ops.hip", "qd_persistent.hip", "qd_batch.hip", "qd_prefill.hip",
+           "qd_capi.hip"]
 ARCH = os.environ.get("QD_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -11,8 +11,8 @@ Mirrors the reference's decode engine: GreedyDecodeEngine.generate
 (evaluation_wrapper.py:149-315) and DecodeCudaGraphRunner
 (evaluation_wrapper.py:747-1005: static input buffers, graph prebuild and
 replay).  The prefill that fills the static KV cache
-(evaluation_wrapper.py:218-228, a full HF forward in the reference) runs here
-as plain PyTorch-ROCm ops in fp32; it is not part of the decode step.
+(evaluation_wrapper.py:218-228, a full HF forward in the reference) is one call
+of the native ``qd_prefill`` (fp32 math on the fp16 matrix cores).
 """
 
 from __future__ import annotations
@@ -150,6 +150,12 @@ class DecodeEngine(_CapturedSteps):
             L.k_cache = self.k_caches[i].data_ptr()
             L.v_cache = self.v_caches[i].data_ptr()
         self._layers = layers
+        # what the descriptor's raw pointers stand for: the native prefill reads
+        # every weight through them
+        self._native_weights = all(
+            t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+            for t in [self.w.embed_tokens, self.w.final_norm_weight] + [t for lw in self.w.layers
+                                                                        for t in lw.tensors().values()])
         d = _lib.ModelDesc()
         d.num_layers = len(self.w.layers)
         d.hidden, d.num_heads, d.num_kv_heads = s.hidden, s.num_heads, s.num_kv_heads
@@ -357,11 +363,12 @@ class DecodeEngine(_CapturedSteps):
     # ------------------------------------------------------------ prefill
     @torch.no_grad()
     def prefill(self, prompt: MultimodalPrompt) -> int:
-        """Causal prefill of the prompt into the static cache (fp32 PyTorch-ROCm ops).
+        """Causal prefill of the prompt into the static cache, in fp32 math.
 
         Follows the text-model loop of transformers Qwen3VLTextModel
         (modeling_qwen3_vl.py:769-852) with M-RoPE positions [3, S]; returns
-        the argmax token of the last position.
+        the argmax token of the last position.  One call of ``qd_prefill``
+        (HIP kernels) where the library takes the shape, else PyTorch-ROCm ops.
         """
         s = self.shape
         dev = self.device
@@ -371,6 +378,33 @@ class DecodeEngine(_CapturedSteps):
         ids = prompt.text_ids
         if ids.numel() and (int(ids.min()) < 0 or int(ids.max()) >= s.vocab):
             raise ValueError(f"prompt token ids outside the vocabulary [0, {s.vocab})")
+        lib = _lib.lib()
+        vis, pos = prompt.vision_embeds, prompt.position_ids
+        nbytes = 0
+        if (self._native_weights and vis.ndim == 2 and vis.shape[1] == s.hidden and ids.ndim == 1
+                and tuple(pos.shape) == (3, S) and not pos.is_floating_point()):
+            nbytes = int(lib.qd_prefill_workspace_bytes(ctypes.byref(self.desc), S))
+        if nbytes == 0:
+            return self._prefill_general(prompt)
+        vis = vis.to(dev)
+        vis = (vis if vis.dtype in (torch.float16, torch.float32) else vis.float()).contiguous()
+        if vis.data_ptr() % 16:
+            vis = vis.clone()
+        ids, pos = ids.to(dev, torch.int64).contiguous(), pos.to(dev, torch.int64).contiguous()
+        token = torch.empty(1, dtype=torch.int64, device=dev)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        with torch.cuda.device(dev):
+            _lib.check(lib.qd_prefill(
+                ctypes.byref(self.desc), _lib.ptr(vis), _lib.QD_F32 if vis.dtype == torch.float32 else _lib.QD_F16,
+                int(vis.shape[0]), _lib.ptr(ids), _lib.ptr(pos), S, _lib.ptr(token), _lib.ptr(ws), nbytes,
+                _lib.stream(dev)), "qd_prefill")
+        return int(token)
+
+    def _prefill_general(self, prompt: MultimodalPrompt) -> int:
+        """The prefill of shapes the kernels do not take, in PyTorch-ROCm ops."""
+        s = self.shape
+        dev = self.device
+        S = prompt.length
         emb = torch.cat([prompt.vision_embeds.to(dev).float(),
                          self.w.embed_tokens[prompt.text_ids.to(dev)].float()], 0)
         pos = prompt.position_ids.to(dev)

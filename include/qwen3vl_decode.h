@@ -499,6 +499,26 @@ int qd_persistent_set_spin_limit(unsigned polls);
  * cuda_decode_gemv_ops/profile.py, are out of scope). */
 int qd_persistent_trace_read(uint64_t* dst, size_t n, int* dims);
 
+/* Prefill of a prompt of `rows` positions at batch 1: n_vision embedding rows
+ * (fp16 or fp32 [n_vision][H]) followed by the rows of text_ids (int64
+ * [rows - n_vision], each in [0, vocab): the caller checks), M-RoPE positions
+ * position_ids (int64 [3][rows], device), causal attention.  Writes cache rows
+ * [0, rows) of every layer of d and the greedy token of the last position
+ * (first index of the largest fp32 logit) to token_out (device int64 [1]).
+ * fp32 math: the fp16 weights meet activations carried as two fp16 values on
+ * the matrix cores, at an error no larger than an fp32 GEMM's.  Uses d's
+ * sizes, weights, inv_freq and caches, not its step state or workspace; the
+ * workspace (256-byte aligned, qd_prefill_workspace_bytes bytes, need not be
+ * zeroed) is the call's own.  qd_prefill_workspace_bytes returns 0 where the
+ * kernels do not apply (head_dim 128, H in {512, 1024, 2048, 3072, 4096, 6144},
+ * I a multiple of 512 up to 16384, Hq a multiple of Hkv with Hq * 128 % 512 == 0,
+ * batch 1).  Replaces the prefill of GreedyDecodeEngine.generate
+ * (evaluation_wrapper.py:218-228). */
+size_t qd_prefill_workspace_bytes(const qd_model_desc* d, int rows);
+int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int n_vision,
+               const int64_t* text_ids, const int64_t* position_ids, int rows, int64_t* token_out,
+               void* workspace, size_t workspace_bytes, void* stream);
+
 /* Synchronously reads the status word of the persistent step, or of the
  * batch step's qkv hand-off (0 = every hand-off completed; bit 0 = a wait
  * exhausted its spin budget, results of that step are invalid) and clears it

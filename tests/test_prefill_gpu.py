@@ -1,0 +1,106 @@
+"""The native prefill (qd_prefill) on the GPU against the oracle's prefill.
+
+Row counts sit at the edges of the kernels' tiles (64 K/V and q rows, 64 / 128 /
+256 GEMM rows, K splits for few rows); shapes cover GQA groups 1, 2 and 4 and
+inputs of very different magnitudes.  The cache holds fp16, so a K/V element may
+be off by half an fp16 step (2^-11 of itself) plus the difference of two fp32
+evaluations, whose sums of 2048 to 6144 terms leave about 3e-6 of a row's rms per
+layer: 2e-5 of the largest value covers the extremes of all elements.
+"""
+
+from __future__ import annotations
+
+import dataclasses
+
+import pytest
+import torch
+
+from oracle import qwen3vl_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SMALL = {"hidden": 512, "num_heads": 4, "num_kv_heads": 4, "intermediate": 512, "vocab": 512}
+GROUP4 = {"hidden": 1024, "num_heads": 8, "num_kv_heads": 2, "intermediate": 1536, "vocab": 512}
+MODEL = {"vocab": 2048}
+
+
+def _check(w, prompt, eng, token):
+    s = w.shape
+    shape = O.OracleShape(**{f.name: getattr(s, f.name) for f in dataclasses.fields(O.OracleShape)})
+    n, cap = prompt.length, eng.capacity
+    caches = [tuple(torch.zeros(1, s.num_kv_heads, cap, 128) for _ in "kv") for _ in range(s.num_layers)]
+    last = O.prefill(w, O.embed_prompt(w, prompt), prompt.position_ids, caches, shape=shape)
+    for li in range(s.num_layers):
+        for got, ref in zip((eng.k_caches[li], eng.v_caches[li]), caches[li]):
+            got = got.cpu().float()
+            assert torch.equal(got[:, :, n:], torch.zeros_like(got[:, :, n:])), "rows past the prompt were written"
+            err, bound = (got - ref).abs(), ref.abs() * 2 ** -11 + 2e-5 * ref.abs().max()
+            print(f"[parity] layer {li}: worst {float((err / bound).max()):.3f} of the bound", flush=True)
+            assert bool((err <= bound).all())
+    logits = O.rms_norm(last, w.final_norm_weight, s.rms_eps) @ w.embed_tokens.float().T
+    assert float(logits.max() - logits[token]) <= 1e-4 * float(logits.abs().max())
+
+
+def _run(case, shape_kw, grid, n_text, layers=2, scale=None):
+    from qwen3vl_hip import _lib, synthetic as syn
+    from qwen3vl_hip.config import Qwen3VLTextShape
+    from qwen3vl_hip.engine import DecodeEngine
+
+    import ctypes
+
+    print(f"case prefill {case}", flush=True)
+    shape = Qwen3VLTextShape(num_layers=layers, **shape_kw)
+    w = syn.model_weights(11, shape)
+    p = syn.multimodal_prompt(11, *((1, *grid) if grid else (0, 0, 0)), n_text, shape=shape)
+    if scale is not None:
+        p = dataclasses.replace(p, vision_embeds=p.vision_embeds.float() * scale(p.vision_embeds.shape[0])[:, None])
+    eng = DecodeEngine(w, capacity=p.length + 5)
+    assert _lib.lib().qd_prefill_workspace_bytes(ctypes.byref(eng.desc), p.length) > 0, "not the native route"
+    token = eng.prefill(p)
+    _check(w, p, eng, token)
+    before = [t.clone() for t in eng.k_caches + eng.v_caches]
+    assert eng.prefill(p) == token
+    assert all(torch.equal(a, b) for a, b in zip(before, eng.k_caches + eng.v_caches)), "a second pass differs"
+    return w, p, eng
+
+
+@pytest.mark.parametrize("n", [1, 2, 16, 17, 63, 64, 65, 127, 129, 257, 513])
+def test_prefill_text_lengths(cuda, n):
+    _run(f"text {n}", MODEL, None, n)
+
+
+@pytest.mark.parametrize("grid,n_text", [((3, 5), 1), ((7, 9), 2), ((24, 32), 330), ((40, 44), 351)])
+def test_prefill_multimodal(cuda, grid, n_text):
+    _run(f"grid {grid} text {n_text}", MODEL, grid, n_text)
+
+
+@pytest.mark.parametrize("kw", [SMALL, GROUP4])
+@pytest.mark.parametrize("n", [1, 70, 200])
+def test_prefill_other_shapes(cuda, kw, n):
+    _run(f"{kw} n={n}", kw, None, n)
+
+
+def test_prefill_rows_of_very_different_magnitude(cuda):
+    """fp32 embedding rows from 1e-4 to 1e4 of the usual size, in one prompt."""
+    _run("scaled rows", MODEL, (8, 11), 9,
+         scale=lambda n: 10.0 ** (torch.arange(n) % 9 - 4).float())
+
+
+def test_prefill_forms_outside_the_native_route(cuda):
+    """Float positions, one position for all rows and float64 embeddings keep
+    their results: the first two by the general path, the last natively."""
+    w, p, eng = _run("forms", SMALL, (2, 3), 4)
+    token, k = eng.prefill(p), [t.clone() for t in eng.k_caches]
+
+    def again(q):
+        for t in eng.k_caches + eng.v_caches:
+            t.zero_()
+        _check(w, dataclasses.replace(q, position_ids=q.position_ids.long().expand(3, q.length)), eng, eng.prefill(q))
+        return eng
+
+    again(dataclasses.replace(p, position_ids=p.position_ids.double()))
+    again(dataclasses.replace(p, position_ids=torch.full((3, 1), 7)))
+    again(dataclasses.replace(p, vision_embeds=p.vision_embeds.double()))
+    assert eng.prefill(p) == token and all(torch.equal(a, b) for a, b in zip(k, eng.k_caches))
+    with pytest.raises(ValueError):
+        eng.prefill(dataclasses.replace(p, text_ids=p.text_ids * 0 + SMALL["vocab"]))
