@@ -1325,8 +1325,9 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
     QD_REQUIRE(w.qkv && w.o_proj && w.gate_up && w.down && w.input_norm && w.post_norm && w.q_norm && w.k_norm &&
                    w.k_cache && w.v_cache,
                QD_ERR_ARG, "layer %d: null pointer", i);
-    QD_REQUIRE(a16(w.qkv) && a16(w.o_proj) && a16(w.gate_up) && a16(w.down) && a16(w.input_norm) && a16(w.post_norm),
-               QD_ERR_ARG, "layer %d: weights must be 16-byte aligned", i);
+    QD_REQUIRE(a16(w.qkv) && a16(w.o_proj) && a16(w.gate_up) && a16(w.down) && a16(w.input_norm) && a16(w.post_norm) &&
+                   aligned(w.k_cache, 8),
+               QD_ERR_ARG, "layer %d: weights must be 16-byte aligned, the K cache 8-byte", i);
     layers[(size_t)i] = qd::PrefillLayer{(const u16*)w.qkv,        (const u16*)w.o_proj,    (const u16*)w.gate_up,
                                          (const u16*)w.down,       (const u16*)w.input_norm, (const u16*)w.post_norm,
                                          (const u16*)w.q_norm,     (const u16*)w.k_norm,    (u16*)w.k_cache,

@@ -395,9 +395,11 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, 
     } else {
       load_act8<float>(hr, k, u[c]);
       float p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      const float* src = part + (long)row * H + k;
+#pragma unroll 4
       for (int i = 0; i < z; ++i) {
         float v[8];
-        load_act8<float>(part + ((long)i * a.S + row) * H, k, v);
+        load_act8<float>(src, (long)i * a.S * H, v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[e] += v[e];
       }
@@ -451,6 +453,7 @@ __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, 
     const long k = (long)c * 2048 + threadIdx.x * 8;
     if (k >= I) continue;
     float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
     for (int i = 0; i < z; ++i) {
       const float* src = a.part + ((long)i * a.S + row) * 2 * I;
       float v[8], w[8];
@@ -482,91 +485,125 @@ __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, 
 }
 
 // Exponent of a head-normalised and rotated vector's image: |x| <= sqrt(2 D) max |w|.
+constexpr float kHeadBound = 16.f;
 __device__ __forceinline__ int head_exp(const uint16_t* w) {
   const int j = lane_id();
-  const float m = wave_max(fmaxf(fabsf(h2f(w[j])), fabsf(h2f(w[j + kHD / 2]))));
-  return split_exp(m * 16.f);
+  return split_exp(wave_max(fmaxf(fabsf(h2f(w[j])), fabsf(h2f(w[j + kHD / 2])))) * kHeadBound);
 }
 
-// Workgroups [0, q/k groups): one wave per (row, q or k head): head RMSNorm,
-// rotation, split image; k also to the cache.  The others: one (kv head, 64
+constexpr int kPrepThreads = 1024;
+
+// Workgroups [0, q/k groups): 16 lanes per (row, q or k head), 4 rotary pairs
+// each: head RMSNorm, rotation, split image; k also to the cache.  The others: one (kv head, 64
 // rows) tile of V each: cache rows, and the split image of the tile transposed,
 // [128 dims][64 rows] with the rows of each half in the order the PV product's
 // operand holds its probabilities in: position 8 g + e is row
-// 16 (e / 4) + 4 g + e % 4.  The tile's exponent goes to vexp and, as the layer's
+// 16 (e / 4) + 4 g + e % 4.  A thread owns one 16-byte chunk of that image, so 8
+// rows of one dim; all its loads are issued before its first store (32 rows a
+// thread, each stored before the next was loaded: 66 us instead of ~9 for 37
+// rows and 8 planes).  The tile's exponent goes to vexp and, as the layer's
 // maximum, to vmax.
-__global__ __launch_bounds__(256) void prefill_qkv_prep_kernel(const PrefillArgs a, const PrefillLayer L, int z,
-                                                               int qk_groups, int layer) {
-  __shared__ float s_red[4];
+__global__ __launch_bounds__(kPrepThreads) void prefill_qkv_prep_kernel(const PrefillArgs a, const PrefillLayer L,
+                                                                        int z, int qk_groups, int layer) {
+  __shared__ float s_red[kPrepThreads / kWave];
   const long NQ = (long)(a.Hq + 2 * a.Hkv) * kHD;
   if ((int)blockIdx.x < qk_groups) {
-    const long item = (long)blockIdx.x * 4 + threadIdx.x / kWave;
+    const long item = (long)blockIdx.x * (kPrepThreads / 16) + threadIdx.x / 16;
     const int heads = a.Hq + a.Hkv;
-    const int row = (int)(item / heads), head = (int)(item % heads);
-    if (row >= a.S) return;
-    const int j = lane_id();
+    const bool live = item < (long)a.S * heads;
+    const int row = live ? (int)(item / heads) : a.S - 1, head = (int)(item % heads);
+    const int j = (lane_id() & 15) * 4;   // dims [j, j + 4) and [64 + j, 64 + j + 4)
     const bool is_q = head < a.Hq;
-    float x0 = 0.f, x1 = 0.f;
-    for (int i = 0; i < z; ++i) {
-      const float* src = a.part + ((long)i * a.S + row) * NQ + (long)head * kHD;
-      x0 += src[j];
-      x1 += src[j + kHD / 2];
-    }
     const uint16_t* nw = is_q ? L.q_norm : L.k_norm;
-    const float2 cs = a.cs[(long)row * (kHD / 2) + j];
-    const float rstd = rsqrtf(wave_sum(x0 * x0 + x1 * x1) / (float)kHD + a.eps);
-    const float n0 = (x0 * rstd) * h2f(nw[j]), n1 = (x1 * rstd) * h2f(nw[j + kHD / 2]);
-    const float o0 = n0 * cs.x - n1 * cs.y, o1 = n1 * cs.x + n0 * cs.y;
-    const int e = head_exp(nw);
-    const float sc = pow2f(-e);
-    _Float16 h0, l0, h1, l1;
-    split2(o0 * sc, h0, l0);
-    split2(o1 * sc, h1, l1);
+    const f32x4* csp = reinterpret_cast<const f32x4*>(a.cs + (long)row * (kHD / 2) + j);
+    const f32x4 cs[2] = {csp[0], csp[1]};
+    float f[2][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[0][e] = h2f(nw[j + e]);
+      f[1][e] = h2f(nw[j + kHD / 2 + e]);
+    }
+    const float* src = a.part + (long)row * NQ + (long)head * kHD + j;
+    f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 4
+    for (int i = 0; i < z; ++i) {
+      x[0] += *reinterpret_cast<const f32x4*>(src + (long)i * a.S * NQ);
+      x[1] += *reinterpret_cast<const f32x4*>(src + (long)i * a.S * NQ + kHD / 2);
+    }
+    float ss = 0.f, mx = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ss = __builtin_fmaf(x[h][e], x[h][e], ss);
+        mx = fmaxf(mx, fabsf(f[h][e]));
+      }
+    const float rstd = rsqrtf(row16_sum(ss) / (float)kHD + a.eps);
+    const float sc = pow2f(-split_exp(row16_max(mx) * kHeadBound));
+    if (!live) return;
+    h4 hi[2], lo[2], kc[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float c = cs[e / 2][2 * (e & 1)], s = cs[e / 2][2 * (e & 1) + 1];
+      const float n0 = (x[0][e] * rstd) * f[0][e], n1 = (x[1][e] * rstd) * f[1][e];
+      const float o[2] = {n0 * c - n1 * s, n1 * c + n0 * s};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        _Float16 a0, b0;
+        split2(o[h] * sc, a0, b0);
+        hi[h][e] = a0;
+        lo[h][e] = b0;
+        kc[h][e] = (_Float16)o[h];
+      }
+    }
     const int hh = is_q ? head : head - a.Hq;
     const long plane = (long)(is_q ? a.Hq : a.Hkv) * a.S * kHD;
-    _Float16* dst = reinterpret_cast<_Float16*>(is_q ? a.q_img : a.k_img) + ((long)hh * a.S + row) * kHD;
-    dst[j] = h0;
-    dst[j + kHD / 2] = h1;
-    dst[plane + j] = l0;
-    dst[plane + j + kHD / 2] = l1;
-    if (!is_q) {
-      uint16_t* kc = L.k_cache + ((long)hh * a.T + row) * kHD;
-      kc[j] = f2h(o0);
-      kc[j + kHD / 2] = f2h(o1);
+    uint16_t* dst = (is_q ? a.q_img : a.k_img) + ((long)hh * a.S + row) * kHD + j;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      *reinterpret_cast<h4*>(dst + h * (kHD / 2)) = hi[h];
+      *reinterpret_cast<h4*>(dst + plane + h * (kHD / 2)) = lo[h];
+      if (!is_q) *reinterpret_cast<h4*>(L.k_cache + ((long)hh * a.T + row) * kHD + j + h * (kHD / 2)) = kc[h];
     }
     return;
   }
   const int tiles = (a.S + kKvTile - 1) / kKvTile;
   const int it = (int)blockIdx.x - qk_groups;
   const int kvh = it / tiles, tile = it % tiles;
-  const int d = threadIdx.x & (kHD - 1), half = threadIdx.x / kHD;
-  const int r0 = tile * kKvTile + half * 32;
-  float v[32];
+  const int d = threadIdx.x & (kHD - 1), chunk = threadIdx.x / kHD;   // chunk = 4 half + g
+  const int r0 = tile * kKvTile + (chunk / 4) * 32 + 4 * (chunk % 4);
+  const float* src = a.part + (long)(a.Hq + a.Hkv + kvh) * kHD + d;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int p = 0; p < z; ++p) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      x[e] = src[((long)p * a.S + min(r0 + 16 * (e / 4) + e % 4, a.S - 1)) * NQ];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += x[e];
+  }
   float mx = 0.f;
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    v[i] = 0.f;
-    if (r0 + i < a.S) {
-      for (int p = 0; p < z; ++p)
-        v[i] += a.part[((long)p * a.S + r0 + i) * NQ + (long)(a.Hq + a.Hkv + kvh) * kHD + d];
-      L.v_cache[((long)kvh * a.T + r0 + i) * kHD + d] = f2h(v[i]);
-      mx = fmaxf(mx, fabsf(v[i]));
+  for (int e = 0; e < 8; ++e) {
+    const int r = r0 + 16 * (e / 4) + e % 4;
+    if (r < a.S) {
+      L.v_cache[((long)kvh * a.T + r) * kHD + d] = f2h(v[e]);
+      mx = fmaxf(mx, fabsf(v[e]));
+    } else {
+      v[e] = 0.f;
     }
   }
-  const int e = split_exp(block_max(mx, s_red, 4));
-  const float sc = pow2f(-e);
+  const int ex = split_exp(block_max(mx, s_red, kPrepThreads / kWave));
+  const float sc = pow2f(-ex);
   const long plane = (long)a.Hkv * tiles * kHD * kKvTile;
-  uint16_t* dst = a.vt_img + ((long)it * kHD + d) * kKvTile + half * 32;
+  uint16_t* dst = a.vt_img + ((long)it * kHD + d) * kKvTile + 8 * chunk;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    float u[8];
-#pragma unroll
-    for (int x = 0; x < 8; ++x) u[x] = v[16 * (x / 4) + 4 * g + x % 4] * sc;
-    store_split8(dst + 8 * g, dst + plane + 8 * g, u);
-  }
+  for (int e = 0; e < 8; ++e) v[e] *= sc;
+  store_split8(dst, dst + plane, v);
   if (threadIdx.x == 0) {
-    a.vexp[it] = e;
-    atomicMax(a.vmax + layer, e);
+    a.vexp[it] = ex;
+    atomicMax(a.vmax + layer, ex);
   }
 }
 
@@ -808,7 +845,8 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
     x.M = a.S; x.N = N; x.K = K;
     return split_gemm_launch(x, g, s);
   };
-  const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + 3) / 4);
+  constexpr int kPrepItems = kPrepThreads / 16;
+  const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + kPrepItems - 1) / kPrepItems);
   // 128 q rows per workgroup once that still gives every CU two workgroups
   const bool wide = (long)((a.S + 127) / 128) * a.Hq >= 2L * qd_host::cu_count();
   const int q_tiles = wide ? (a.S + 127) / 128 : (a.S + 63) / 64;
@@ -821,7 +859,8 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
                          L.input_norm, 0);
     if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
     if ((st = gemm(L.qkv, a.scale, 1, qn, a.H, p.qkv))) return st;
-    hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)), dim3(256), 0, s, a, L,
+    hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)),
+                       dim3(kPrepThreads), 0, s, a, L,
                        p.qkv.z, qk_groups, li);
     if ((st = qd_host::launch_status("prefill_qkv_prep_kernel"))) return st;
     if (wide)
