@@ -1083,7 +1083,7 @@ int qd_decode_status(const qd_model_desc* d, unsigned* status, int reset) {
   size_t total = 0;
   step_layout(d, splits_of(d), &b, &total);
   hipError_t e = hipMemcpy(status, b.control, sizeof(unsigned), hipMemcpyDeviceToHost);
-  if (e == hipSuccess && reset) {
+  if (e == hipSuccess && reset && *status != 0) {   // a clear word needs no second transfer
     const unsigned zero = 0;
     e = hipMemcpy(b.control, &zero, sizeof(unsigned), hipMemcpyHostToDevice);
   }
@@ -1190,6 +1190,21 @@ int qd_decode_advance(const int64_t* token, int64_t* out_tokens, int64_t* counte
   QD_REQUIRE(token && counter && cache_position && rope_position, QD_ERR_ARG, "null pointer");
   return qd::decode_advance_launch(token, out_tokens, counter, cache_position, rope_position, max_tokens,
                                    S(stream));
+}
+
+int qd_decode_set_state(int64_t* token, int64_t* cache_position, int64_t* rope_position, int64_t* counter,
+                        const int64_t* tokens, const int64_t* cache_positions, const int64_t* rope_positions, int batch,
+                        void* stream) {
+  QD_REQUIRE(token && cache_position && rope_position && tokens && cache_positions && rope_positions, QD_ERR_ARG,
+             "null pointer");
+  QD_REQUIRE(batch >= 1 && batch <= qd::kBatchMax, QD_ERR_SHAPE, "batch %d outside 1..%d", batch, qd::kBatchMax);
+  qd::DecodeState v;
+  for (int b = 0; b < batch; ++b) {
+    v.token[b] = tokens[b];
+    v.cache_position[b] = cache_positions[b];
+    v.rope_position[b] = rope_positions[b];
+  }
+  return qd::decode_set_state_launch(token, cache_position, rope_position, counter, v, batch, S(stream));
 }
 
 int qd_decode_advance_batch(const int64_t* token, int64_t* out_tokens, int64_t* counter, int64_t* cache_position,

@@ -168,6 +168,13 @@ int embed_gather_launch(const uint16_t* table, const int64_t* token, float* out,
 int decode_advance_launch(const int64_t* token, int64_t* out_tokens, int64_t* counter, int64_t* cache_position,
                           int64_t* rope_position, int max_tokens, hipStream_t s);
 
+// Host values of a decode call's device state (up to 8 sequences).
+struct DecodeState {
+  int64_t token[8], cache_position[8], rope_position[8];
+};
+int decode_set_state_launch(int64_t* token, int64_t* cache_position, int64_t* rope_position, int64_t* counter,
+                            const DecodeState& v, int batch, hipStream_t s);
+
 // ---------------------------------------------------------------- persistent step
 
 constexpr int kPersistMaxLayers = 32;

@@ -241,4 +241,27 @@ int decode_advance_launch(const int64_t* token, int64_t* out_tokens, int64_t* co
   return qd_host::launch_status("decode_advance_kernel");
 }
 
+// The state of a decode call, the values in the kernel arguments: one launch
+// where a fill per word (batch 1) or a host copy per tensor (batch, each a
+// synchronous transfer) took 4 and 3.
+__global__ void decode_set_state_kernel(int64_t* token, int64_t* cache_position, int64_t* rope_position,
+                                        int64_t* counter, const DecodeState v, int batch) {
+  const int b = threadIdx.x;
+  if (b < batch) {
+    token[b] = v.token[b];
+    cache_position[b] = v.cache_position[b];
+    rope_position[3 * b + 0] = v.rope_position[b];
+    rope_position[3 * b + 1] = v.rope_position[b];
+    rope_position[3 * b + 2] = v.rope_position[b];
+  }
+  if (b == 0 && counter != nullptr) counter[0] = 0;
+}
+
+int decode_set_state_launch(int64_t* token, int64_t* cache_position, int64_t* rope_position, int64_t* counter,
+                            const DecodeState& v, int batch, hipStream_t s) {
+  hipLaunchKernelGGL(decode_set_state_kernel, dim3(1), dim3(64), 0, s, token, cache_position, rope_position, counter, v,
+                     batch);
+  return qd_host::launch_status("decode_set_state_kernel");
+}
+
 }  // namespace qd

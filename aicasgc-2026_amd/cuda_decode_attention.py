@@ -19,6 +19,8 @@ splits to fill 256 CUs (results do not depend on the split count).
 
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
 from qwen3vl_hip import _lib
@@ -31,33 +33,43 @@ def _load_ext():
 
 
 def _supported(q, k, v, num_key_value_groups, cache_position) -> bool:
-    return not (
-        q.device.type != "cuda" or k.device.type != "cuda" or v.device.type != "cuda"
-        or cache_position.device.type != "cuda"
-        or q.dtype != torch.float16 or k.dtype != torch.float16 or v.dtype != torch.float16
-        or q.ndim != 4 or k.ndim != 4 or v.ndim != 4
-        or q.shape[0] != 1 or q.shape[2] != 1 or q.shape[-1] != 128
-        or k.shape[0] != 1 or k.shape != v.shape or k.shape[-1] != 128
-        or k.shape[1] * num_key_value_groups != q.shape[1]
-        or num_key_value_groups not in (1, 2, 4)
-        or q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1
-        or k.stride(1) != v.stride(1) or k.stride(2) != v.stride(2)
-        or q.stride(1) % 8 != 0 or k.stride(1) % 8 != 0 or k.stride(2) % 8 != 0
-        or q.data_ptr() % 16 != 0 or k.data_ptr() % 16 != 0 or v.data_ptr() % 16 != 0
-        or cache_position.dtype != torch.long or cache_position.numel() != 1
-    )
+    if not (q.is_cuda and k.is_cuda and v.is_cuda and cache_position.is_cuda):
+        return False
+    half = torch.float16
+    if q.dtype != half or k.dtype != half or v.dtype != half or cache_position.dtype != torch.long:
+        return False
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if (len(qs) != 4 or len(ks) != 4 or ks != vs or qs[0] != 1 or qs[2] != 1 or qs[3] != 128 or ks[0] != 1
+            or ks[3] != 128 or num_key_value_groups not in (1, 2, 4) or ks[1] * num_key_value_groups != qs[1]
+            or cache_position.numel() != 1):
+        return False
+    qt, kt, vt = q.stride(), k.stride(), v.stride()
+    if (qt[3] != 1 or kt[3] != 1 or vt[3] != 1 or kt[1] != vt[1] or kt[2] != vt[2]
+            or qt[1] % 8 or kt[1] % 8 or kt[2] % 8):
+        return False
+    return not (q.data_ptr() % 16 or k.data_ptr() % 16 or v.data_ptr() % 16)
+
+
+@lru_cache(maxsize=1024)
+def _default_splits(seq_len: int) -> int:
+    return int(_load_ext().qd_attention_default_splits(seq_len))
 
 
 def _splits(seq_len: int, split_k: int | None) -> int:
-    s = int(_load_ext().qd_attention_default_splits(int(seq_len)))
+    s = _default_splits(int(seq_len))
     return max(s, int(split_k)) if split_k else s
+
+
+@lru_cache(maxsize=1024)
+def _ws_bytes(hq: int, hkv: int, n_split: int) -> int:
+    return int(_load_ext().qd_attention_workspace_bytes(hq, hkv, n_split))
 
 
 def _out_buffer(workspace, q) -> torch.Tensor:
     hq, d = q.shape[1], q.shape[-1]
-    if (workspace is not None and "out" in workspace and tuple(workspace["out"].shape) == (1, hq, d)
-            and workspace["out"].dtype == q.dtype and workspace["out"].device == q.device):
-        return workspace["out"]
+    t = workspace.get("out") if workspace is not None else None
+    if t is not None and t.shape == (1, hq, d) and t.dtype == q.dtype and t.device == q.device:
+        return t
     return torch.empty((1, hq, d), dtype=q.dtype, device=q.device)
 
 
@@ -80,12 +92,12 @@ def _run_fused(q, k, v, scaling, num_key_value_groups, cache_position, split_k, 
     hq, hkv, T = q.shape[1], k.shape[1], k.shape[2]
     n_split = _splits(T, split_k)
     out = _out_buffer(workspace, q)
-    ws = _ws_buffer(workspace, q, int(lib.qd_attention_workspace_bytes(hq, hkv, n_split)))
+    ws = _ws_buffer(workspace, q, _ws_bytes(hq, hkv, n_split))
     _lib.check(lib.qd_attention_decode(
         _lib.ptr(q), _lib.QD_F16, q.stride(1), _lib.ptr(k), _lib.ptr(v), k.stride(1), k.stride(2), T,
         _lib.ptr(cache_position), float(scaling), _lib.ptr(out), _lib.QD_F16, hq, hkv, n_split, _lib.ptr(ws),
         _lib.stream(q.device)), "qd_attention_decode")
-    return out.unsqueeze(2).transpose(1, 2)
+    return out.unsqueeze(1)
 
 
 def _qkv_rope_attention(qkv, q_weight, k_weight, eps: float, cos, sin, k_cache, v_cache, scaling, cache_position,
@@ -118,14 +130,14 @@ def _qkv_rope_attention(qkv, q_weight, k_weight, eps: float, cos, sin, k_cache, 
     lib = _load_ext()
     n_split = _splits(T, split_k)
     out = _out_buffer(workspace, qkv.view(1, hq + 2 * hkv, 1, 128)[:, :hq])
-    ws = _ws_buffer(workspace, qkv, int(lib.qd_attention_workspace_bytes(hq, hkv, n_split)))
+    ws = _ws_buffer(workspace, qkv, _ws_bytes(hq, hkv, n_split))
     qw, kw = q_weight.contiguous(), k_weight.contiguous()   # held until the launch is enqueued
     cs, sn, cp = cos.contiguous(), sin.contiguous(), cache_position.contiguous()
     _lib.check(lib.qd_attention_qkv_decode_f16(
         _lib.ptr(qkv), _lib.ptr(qw), _lib.ptr(kw), float(eps), _lib.ptr(cs), _lib.ptr(sn), _lib.ptr(k_cache),
         _lib.ptr(v_cache), k_cache.stride(1), k_cache.stride(2), T, _lib.ptr(cp), float(scaling), _lib.ptr(out),
         hq, hkv, n_split, _lib.ptr(ws), _lib.stream(qkv.device)), "qd_attention_qkv_decode_f16")
-    return out.unsqueeze(2).transpose(1, 2)
+    return out.unsqueeze(1)
 
 
 def decode_attn_v4_cta_qhead_splitkv_fused(q, k, v, scaling, num_key_value_groups, cache_position, split_k: int = 4,
@@ -184,7 +196,7 @@ def decode_attn_v4_splitkv(q, k, v, scaling, num_key_value_groups, cache_positio
         "qd_attention_partial")
     _lib.check(lib.qd_attention_merge(_lib.ptr(o_part), _lib.ptr(lse), _lib.ptr(out), _lib.QD_F16, hq, n_split, st),
                "qd_attention_merge")
-    return out.unsqueeze(2).transpose(1, 2)
+    return out.unsqueeze(1)
 
 
 def grouped_prefix_cachepos_splitkv(q, k, v, scaling, num_key_value_groups, cache_position, split_k: int,

@@ -16,7 +16,7 @@ import torch
 from qwen3vl_hip import _lib
 
 from .matvec import nosplit_matvec_half
-from .runtime import _check, _contig_weight, _load_ext, _p, _require_decode_half, _reuse, _stream
+from .runtime import _check, _contig_weight, _flat, _load_ext, _p, _require_decode_half, _reuse, _stream
 
 __all__ = [
     "fused_add_rmsnorm_gateup_half", "fused_rmsnorm_qkv_half", "fused_silu_downproj_half",
@@ -29,10 +29,6 @@ __all__ = [
 ]
 
 
-def _vec(t: torch.Tensor) -> torch.Tensor:
-    return t.reshape(-1).contiguous()
-
-
 def fused_rmsnorm_qkv_half(x: torch.Tensor, norm_weight: torch.Tensor, weight: torch.Tensor,
                            bias: torch.Tensor | None, eps: float) -> torch.Tensor:
     """out = W (rmsnorm(x) * gamma) (+ b)  (reference fused.py:71-105)."""
@@ -40,14 +36,14 @@ def fused_rmsnorm_qkv_half(x: torch.Tensor, norm_weight: torch.Tensor, weight: t
     _require_decode_half(name, x, norm_weight, weight, x=x)
     w = _contig_weight(weight, name)
     n, k = w.shape
-    x_vec, g = _vec(x), _vec(norm_weight)
+    x_vec, g = _flat(x), _flat(norm_weight)
     if x_vec.numel() != k or g.numel() != k:
         raise RuntimeError(f"{name}: x/norm_weight must have K={k} elements")
-    out = torch.empty((n,), dtype=x.dtype, device=x.device)
-    b = _vec(bias) if bias is not None else None
+    out = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    b = _flat(bias) if bias is not None else None
     _check(_load_ext().qd_rmsnorm_matvec_f16(_p(x_vec), _p(g), _p(w), _p(b), _p(out), n, k, float(eps),
                                              _stream(x)), name)
-    return out.view(*x.shape[:-1], n)
+    return out
 
 
 def fused_add_rmsnorm_gateup_half(residual: torch.Tensor, x: torch.Tensor, norm_weight: torch.Tensor,
@@ -62,8 +58,8 @@ def fused_add_rmsnorm_gateup_half(residual: torch.Tensor, x: torch.Tensor, norm_
     n, k = w.shape
     res_out = _reuse(workspace, "fused_add_rmsnorm_gateup", "residual_out", (k,), residual.dtype, residual.device)
     out = _reuse(workspace, "fused_add_rmsnorm_gateup", "out", (n,), residual.dtype, residual.device)
-    b = _vec(bias) if bias is not None else None
-    rv, xv, gv = _vec(residual), _vec(x), _vec(norm_weight)   # held until the launch is enqueued
+    b = _flat(bias) if bias is not None else None
+    rv, xv, gv = _flat(residual), _flat(x), _flat(norm_weight)   # held until the launch is enqueued
     _check(_load_ext().qd_add_rmsnorm_matvec_f16(_p(rv), _p(xv), _p(gv), _p(w), _p(b), _p(res_out), _p(out), n, k,
                                                  float(eps), _stream(x)), name)
     return res_out.view_as(residual), out.view(*residual.shape[:-1], n)
@@ -76,11 +72,11 @@ def fused_silu_downproj_half(gate_up: torch.Tensor, weight: torch.Tensor, bias: 
     _require_decode_half(name, gate_up, weight, x=gate_up)
     w = _contig_weight(weight, name)
     n, k = w.shape
-    gu = _vec(gate_up)
+    gu = _flat(gate_up)
     if gu.numel() != 2 * k:
         raise RuntimeError(f"{name}: gate_up must have 2*K = {2 * k} elements")
     out = _reuse(workspace, "fused_silu_downproj", "out", (n,), gate_up.dtype, gate_up.device)
-    b = _vec(bias) if bias is not None else None
+    b = _flat(bias) if bias is not None else None
     _check(_load_ext().qd_silu_matvec_f16(_p(gu), _p(w), _p(b), _p(out), n, k, _stream(gate_up)), name)
     return out.view(*gate_up.shape[:-1], n)
 
@@ -91,12 +87,12 @@ def _gateup_silu_down(name: str, x, gate_up_weight, down_proj_weight, bias, work
     wd = _contig_weight(down_proj_weight, name)
     two_i, h = wgu.shape
     n, i = wd.shape
-    if two_i != 2 * i or _vec(x).numel() != h:
+    if two_i != 2 * i or x.numel() != h:
         raise RuntimeError(f"{name}: inconsistent shapes gate_up {tuple(wgu.shape)} down {tuple(wd.shape)}")
     hidden = _reuse(workspace, kind, "hidden_out", (i,), x.dtype, x.device)
     out = _reuse(workspace, kind, "out", (n,), x.dtype, x.device)
-    b = _vec(bias) if bias is not None else None
-    xv = _vec(x)
+    b = _flat(bias) if bias is not None else None
+    xv = _flat(x)
     _check(_load_ext().qd_gateup_silu_down_f16(_p(xv), _p(wgu), _p(wd), _p(b), _p(hidden), _p(out), h, i,
                                                _stream(x)), name)
     return hidden.view(*x.shape[:-1], i), out.view(*x.shape[:-1], n)
@@ -150,8 +146,8 @@ def _post_attn_mlp(name, residual, attn_output, norm_weight, gate_up_weight, dow
         raise RuntimeError(f"{name}: inconsistent shapes")
     hidden = _reuse(workspace, kind, "hidden_out", (i,), residual.dtype, residual.device)
     out = _reuse(workspace, kind, "out", (n,), residual.dtype, residual.device)
-    b = _vec(bias) if bias is not None else None
-    rv, av, gv = _vec(residual), _vec(attn_output), _vec(norm_weight)   # held until the launch is enqueued
+    b = _flat(bias) if bias is not None else None
+    rv, av, gv = _flat(residual), _flat(attn_output), _flat(norm_weight)   # held until the launch is enqueued
     if next_position is None:
         _check(_load_ext().qd_post_attn_mlp_f16(_p(rv), _p(av), _p(gv), _p(wgu), _p(wd), _p(b), _p(hidden), _p(out),
                                                 h, i, float(eps), _stream(residual)), name)

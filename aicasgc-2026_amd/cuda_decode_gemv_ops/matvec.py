@@ -12,7 +12,7 @@ import torch
 
 from qwen3vl_hip import _lib
 
-from .runtime import NOSPLIT_VARIANTS, _check, _contig_weight, _load_ext, _p, _require_decode_half, _reuse, _stream
+from .runtime import NOSPLIT_VARIANTS, _check, _contig_weight, _flat, _load_ext, _p, _require_decode_half, _reuse, _stream
 
 __all__ = [
     "splitk_matvec", "splitk_matvec_row4", "splitk_matvec_row8_shared", "splitk_matvec_row4_shared_vec_half",
@@ -31,14 +31,14 @@ def _matvec(name: str, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor
         _require_decode_half(name, bias)
     w = _contig_weight(weight, name)
     n, k = w.shape
-    x_vec = x.reshape(-1).contiguous()
+    x_vec = _flat(x)
     if x_vec.numel() != k:
         raise RuntimeError(f"{name}: x has {x_vec.numel()} elements, weight expects K={k}")
-    if out_vec is None:
-        out_vec = torch.empty((n,), dtype=x.dtype, device=x.device)
-    b = bias.reshape(-1).contiguous() if bias is not None else None
-    _check(_load_ext().qd_matvec_f16(_p(x_vec), _p(w), _p(b), _p(out_vec), n, k, _stream(x)), name)
-    return out_vec.view(*x.shape[:-1], n)
+    shape = (*x.shape[:-1], n)
+    out = torch.empty(shape, dtype=x.dtype, device=x.device) if out_vec is None else out_vec.view(shape)
+    b = _flat(bias) if bias is not None else None
+    _check(_load_ext().qd_matvec_f16(_p(x_vec), _p(w), _p(b), _p(out), n, k, _stream(x)), name)
+    return out
 
 
 def nosplit_matvec_half(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,

@@ -59,7 +59,7 @@ def _check(status: int, what: str) -> None:
 def _require_decode_half(name: str, *tensors: torch.Tensor, x: torch.Tensor | None = None) -> None:
     """The reference's guard: fp16 GPU tensors, single-token decode shape."""
     for t in tensors:
-        if t.device.type != "cuda" or t.dtype != torch.float16:
+        if not t.is_cuda or t.dtype != torch.float16:
             raise RuntimeError(f"{name} expects fp16 CUDA single-token decode tensors")
     if x is not None and (x.ndim < 2 or x.shape[-2] != 1):
         raise RuntimeError(f"{name} expects fp16 CUDA single-token decode tensors")
@@ -73,8 +73,14 @@ def _contig_weight(w: torch.Tensor, name: str) -> torch.Tensor:
 
 def _reuse(workspace: dict | None, kind: str, key: str, shape: tuple, dtype, device) -> torch.Tensor:
     """Workspace reuse with the reference's dict convention (fused.py:294-318)."""
-    if (workspace is not None and workspace.get("type") == kind and key in workspace
-            and tuple(workspace[key].shape) == shape and workspace[key].dtype == dtype
-            and workspace[key].device == device):
-        return workspace[key]
+    if workspace is not None and workspace.get("type") == kind:
+        t = workspace.get(key)
+        if t is not None and t.shape == shape and t.dtype == dtype and t.device == device:
+            return t
     return torch.empty(shape, dtype=dtype, device=device)
+
+
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    """``t`` itself when its elements already lie in order, else a contiguous
+    copy: only its pointer and element count are used."""
+    return t if t.is_contiguous() else t.contiguous()

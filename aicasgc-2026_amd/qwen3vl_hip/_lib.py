@@ -30,6 +30,7 @@ STEP_AUTO, STEP_CHAIN, STEP_PERSISTENT = 0, 1, 2
 QD_ERR_ARG, QD_ERR_SHAPE = -1, -2
 
 P = c_void_p
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 # name -> (restype, argtypes)
 _SIGS = {
@@ -84,6 +85,7 @@ _SIGS = {
     "qd_batch_tile_rows": (c_int, [c_long, c_long, c_int]),
     "qd_batch_gemv": (c_int, [P, c_long, P, c_float, P, c_long, c_long, c_long, c_long, P, c_long, P, c_long, c_int,
                               c_int, P, ctypes.c_size_t, P]),
+    "qd_decode_set_state": (c_int, [P, P, P, P, POINTER(c_int64), POINTER(c_int64), POINTER(c_int64), c_int, P]),
     "qd_decode_advance_batch": (c_int, [P, P, P, P, P, c_int, c_int, P]),
 }
 
@@ -114,12 +116,16 @@ def check(status: int, what: str) -> None:
         raise RuntimeError(f"{what} failed with status {status}: {last_error()}")
 
 
+# Plain ints for the c_void_p parameters: a decode call passes up to 20 of them
+# and a c_void_p object for each costs more than the pointer itself.
 def ptr(t: torch.Tensor | None):
-    return None if t is None else c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def stream(device: torch.device | None = None):
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def stream(device: torch.device | None = None) -> int:
+    """The current stream of ``device`` (default: the current device) as a pointer."""
+    index = None if device is None else device.index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def call(name: str, *args) -> None:

@@ -33,6 +33,18 @@ def rope_inv_freq(shape: Qwen3VLTextShape = QWEN3VL_2B) -> torch.Tensor:
     return 1.0 / (shape.rope_theta ** (torch.arange(0, d, 2, dtype=torch.float32) / d))
 
 
+def _host_ints(x, n: int):
+    """The n values of a list, a tuple, a number or a CPU tensor as a ctypes
+    int64 array, or None for anything else (a device tensor stays there)."""
+    if torch.is_tensor(x):
+        if x.is_cuda:
+            return None
+        x = x.reshape(-1).tolist()
+    elif not isinstance(x, (list, tuple)):
+        x = [x]
+    return (ctypes.c_int64 * n)(*(int(v) for v in x)) if len(x) == n else None
+
+
 class _CapturedSteps:
     """HIP-graph capture shared by the engines: one step (``step_eager``:
     decode + advance) in one graph, and k consecutive steps in one graph for
@@ -42,6 +54,18 @@ class _CapturedSteps:
     most steps_per_graph steps per replay), and each replay's launch gap (a
     single-step replay costs ~8 us more than a step inside a longer graph) is
     paid once per replay."""
+
+    def _set_state(self, tokens, cache_positions, rope_positions, batch: int, zero_counter: bool) -> bool:
+        """The step state from host values in one launch; False when some are on the device."""
+        v = [_host_ints(x, batch) for x in (tokens, cache_positions, rope_positions)]
+        if any(x is None for x in v):
+            return False
+        with torch.cuda.device(self.device):
+            _lib.check(_lib.lib().qd_decode_set_state(
+                _lib.ptr(self.token), _lib.ptr(self.cache_position), _lib.ptr(self.rope_position),
+                _lib.ptr(self.step_counter) if zero_counter else None, *v, batch, _lib.stream(self.device)),
+                "qd_decode_set_state")
+        return True
 
     def _state_tensors(self):
         return (self.token, self.cache_position, self.rope_position, self.step_counter)
@@ -210,9 +234,7 @@ class DecodeEngine(_CapturedSteps):
 
     # ------------------------------------------------------------ state
     def set_state(self, token: int, cache_position: int, rope_position: int) -> None:
-        self.token.fill_(int(token))
-        self.cache_position.fill_(int(cache_position))
-        self.rope_position.fill_(int(rope_position))
+        self._set_state(int(token), int(cache_position), int(rope_position), 1, False)
 
     def reserve_tokens(self, n: int) -> None:
         if self.out_tokens.numel() < n:
@@ -298,8 +320,7 @@ class DecodeEngine(_CapturedSteps):
         if start_position + n_steps > self.capacity:
             raise ValueError("static cache too small for the requested generation")
         self.reserve_tokens(n_steps)
-        self.set_state(first_token, start_position, start_position + rope_delta)
-        self.step_counter.zero_()
+        self._set_state(int(first_token), int(start_position), int(start_position + rope_delta), 1, True)
         if eos_token_ids is not None and n_steps > 0:
             n_out = self._decode_until_eos(n_steps, use_graph, set(int(t) for t in eos_token_ids),
                                            max(1, int(eos_window)))
@@ -565,6 +586,8 @@ class BatchDecodeEngine(_CapturedSteps):
         d.advance_max_tokens = int(self.out_tokens.shape[0])
 
     def set_state(self, tokens, cache_positions, rope_positions) -> None:
+        if self._set_state(tokens, cache_positions, rope_positions, self.batch, False):
+            return
         self.token.copy_(torch.as_tensor(tokens, dtype=torch.int64))
         self.cache_position.copy_(torch.as_tensor(cache_positions, dtype=torch.int64))
         rp = torch.as_tensor(rope_positions, dtype=torch.int64).view(-1, 1).expand(self.batch, 3)
@@ -620,8 +643,9 @@ class BatchDecodeEngine(_CapturedSteps):
         if min(int(t) for t in first_tokens) < 0 or max(int(t) for t in first_tokens) >= self.shape.vocab:
             raise ValueError("token ids outside the vocabulary")
         self.reserve_tokens(n_steps)
-        self.set_state(first_tokens, start_positions, rope_positions)
-        self.step_counter.zero_()
+        if not self._set_state(first_tokens, start_positions, rope_positions, self.batch, True):
+            self.set_state(first_tokens, start_positions, rope_positions)
+            self.step_counter.zero_()
         if use_graph:
             self.replay_steps(n_steps)
         else:

@@ -554,6 +554,15 @@ int qd_batch_gemv(const float* x, long ldx, const void* gamma, float eps, const 
  * layout (qd_model_desc.batch_tiled_weights); 0 for sizes <= 0. */
 int qd_batch_tile_rows(long rows, long K, int silu);
 
+/* Sets the device state of a decode call from host values, in one launch:
+ * token[b], cache_position[b] and the three rope_position[b] words of each of
+ * the batch (1..8) sequences (the host arrays are read before the call
+ * returns), and, when counter != NULL, counter[0] = 0.  Replaces the input
+ * buffer writes of DecodeCudaGraphRunner (evaluation_wrapper.py:941-960). */
+int qd_decode_set_state(int64_t* token, int64_t* cache_position, int64_t* rope_position,
+                        int64_t* counter, const int64_t* tokens, const int64_t* cache_positions,
+                        const int64_t* rope_positions, int batch, void* stream);
+
 /* qd_decode_advance for a batch: out_tokens [max_tokens][batch]. */
 int qd_decode_advance_batch(const int64_t* token, int64_t* out_tokens, int64_t* counter,
                             int64_t* cache_position, int64_t* rope_position, int max_tokens, int batch,

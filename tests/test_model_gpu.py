@@ -92,3 +92,22 @@ def test_full_model_config3_first_64_tokens(cuda, config3_weights, step_mode):
     print(f"first mismatch: {first_bad}; margins there: "
           f"{gold['margins'][first_bad] if first_bad is not None else None}", flush=True)
     assert toks == ref
+
+
+@pytest.mark.parametrize("form", ["lists", "cpu tensors", "device tensors", "one for all"])
+def test_batch_state_forms(cuda, form):
+    """The step state set from host values in one launch, from device tensors, or broadcast."""
+    from qwen3vl_hip import synthetic as syn
+    from qwen3vl_hip.config import Qwen3VLTextShape
+    from qwen3vl_hip.engine import BatchDecodeEngine
+
+    eng = BatchDecodeEngine(syn.model_weights(3, Qwen3VLTextShape(num_layers=1, vocab=512)), 3, 16)
+    vals = ([7, 8, 9], [1, 2, 3], [4, 5, 6]) if form != "one for all" else ([7], [2], [5])
+    want = [v * (3 // len(v)) for v in vals]
+    if "tensors" in form:
+        vals = tuple(torch.tensor(v, device=cuda if form.startswith("device") else "cpu") for v in vals)
+    eng.step_counter.fill_(5)
+    eng.set_state(*vals)
+    assert eng.token.tolist() == want[0] and eng.cache_position.tolist() == want[1]
+    assert eng.rope_position.tolist() == [[p] * 3 for p in want[2]]
+    assert int(eng.step_counter) == 5
