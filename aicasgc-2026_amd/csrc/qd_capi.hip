@@ -1284,7 +1284,9 @@ size_t prefill_layout(const qd_model_desc* d, long S_, qd::PrefillPlan* plan, Pr
   // 32-bit byte offsets into the GEMM operands
   if ((kmax * S_ * 2) >> 32 || (nmax * kmax * 2) >> 32 || S_ * (Hq + Hkv) >> 31) return 0;
   *plan = qd::prefill_plan(S_, (int)H, (int)Hq, (int)Hkv, (int)I);
-  if (plan->qkv.tile < 0 || plan->o_proj.tile < 0 || plan->gate_up.tile < 0 || plan->down.tile < 0) return 0;
+  if (plan->qkv.tile < 0) return 0;
+  for (int l = 0; l < 2; ++l)
+    if (plan->o_proj[l].tile < 0 || plan->gate_up[l].tile < 0 || plan->down[l].tile < 0) return 0;
   const long tiles = (S_ + 63) / 64;
   size_t off = 0;
   auto take = [&](size_t n) {

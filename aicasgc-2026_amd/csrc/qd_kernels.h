@@ -374,7 +374,7 @@ struct PrefillArgs {
   unsigned* argmax_count;         // [64] cleared for the lm_head
 };
 struct PrefillPlan {
-  GemmPlan qkv, o_proj, gate_up, down;
+  GemmPlan qkv, o_proj[2], gate_up[2], down[2];   // [1]: the last layer's, of the last row alone
   long part_floats;
 };
 PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I);

@@ -43,6 +43,8 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kHD = 128;        // head dim
 constexpr int kKvTile = 64;     // K/V rows per attention tile
@@ -285,18 +287,20 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
 
 namespace {
 
-// Tile shapes and their cost: a workgroup's microseconds per 1024 of K with
-// every CU busy (measured, S = 1024 and 4001 at the 2B shapes) and how many
-// share a CU.
+// Tile shapes, 8 waves each (4 along m, 2 along n: a wave's W rows are read from
+// LDS once for both planes, so wide wave tiles read least), and their cost: a
+// workgroup's microseconds per 1024 of K with every CU busy, beside ~3 us of
+// ramp, and how many share a CU.  Measured at the 2B shapes (MFMA rate):
+// 344 us (1169 TFLOP/s) at 4001 x 12288 x 2048 on 256 x 256, 177 us (1140) at
+// 4001 x 2048 x 6144 on 128 x 256, 35 us (975) at 1024 x 4096 x 2048 on
+// 128 x 128, where four waves of 64 x 64 took 40.
 struct GemmTile {
   int bm, bn, bk, per_cu;
   float us;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {256, 256, 32, 1, 57.f},   // 1144 TFLOP/s of MFMA at 4001 x 12288 x 2048
-    {128, 128, 64, 1, 20.f},   // 824 at 1024 x 4096 x 2048
-    {64, 128, 64, 1, 13.f},
-    {64, 64, 64, 2, 13.f},
+    {256, 256, 32, 1, 57.f}, {128, 256, 32, 1, 29.f},  {128, 128, 64, 1, 16.f},
+    {64, 128, 64, 1, 11.f}, {64, 64, 64, 2, 12.f},
 };
 
 template <int BM, int BN, int BK, int WM, int WN>
@@ -321,7 +325,9 @@ GemmPlan split_gemm_plan(long M, long N, long K) {
       if (K % ((long)g.bk * z) != 0) break;
       const long wgs = ((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn) * z;
       const long rounds = (wgs + (long)cus * g.per_cu - 1) / ((long)cus * g.per_cu);
-      const float us = (float)rounds * (3.f + g.us * (float)(K / z) / 1024.f) +
+      // a grid that leaves CUs idle runs each workgroup faster (64 / 192 of 256 CUs: 0.72 / 0.82)
+      const float fill = (float)wgs / (float)(rounds * cus * g.per_cu);
+      const float us = (float)rounds * (3.f + (0.7f + 0.3f * fill * fill) * g.us * (float)(K / z) / 1024.f) +
                        8.f * (float)z * (float)M * (float)N / 4e6f;
       if (best.tile < 0 || us < best_us) {
         best = GemmPlan{c, z};
@@ -338,10 +344,11 @@ int split_gemm_launch(const SplitGemmArgs& a, const GemmPlan& p, hipStream_t s) 
   // 32-bit byte offsets into the operands
   if ((size_t)a.M * a.K * 2 >> 32 || (size_t)a.N * a.K * 2 >> 32) return QD_ERR_SHAPE;
   switch (p.tile) {
-    case 0: return launch_gemm<256, 256, 32, 2, 4>(a, p.z, s);
-    case 1: return launch_gemm<128, 128, 64, 2, 2>(a, p.z, s);
-    case 2: return launch_gemm<64, 128, 64, 2, 2>(a, p.z, s);
-    default: return launch_gemm<64, 64, 64, 2, 2>(a, p.z, s);
+    case 0: return launch_gemm<256, 256, 32, 4, 2>(a, p.z, s);
+    case 1: return launch_gemm<128, 256, 32, 4, 2>(a, p.z, s);
+    case 2: return launch_gemm<128, 128, 64, 4, 2>(a, p.z, s);
+    case 3: return launch_gemm<64, 128, 64, 4, 2>(a, p.z, s);
+    default: return launch_gemm<64, 64, 64, 4, 2>(a, p.z, s);
   }
 }
 
@@ -367,14 +374,16 @@ __global__ __launch_bounds__(256) void prefill_init_kernel(const PrefillArgs a) 
 
 constexpr int kRowChunks = 4;   // 8-value chunks per thread of a row: H up to 8192
 
-// One row per workgroup: h[row] (+ the GEMM's z partial rows, or the prompt's
-// embedding instead, layer 0), RMSNorm, split image and its scale.  HBM / L2
-// bound: reads (z + 1) and writes 2 x 4 bytes per value.
+// One row per workgroup, rows row0 .. row0 + grid: h[row] (+ the GEMM's z
+// partial rows, or the prompt's embedding instead, layer 0), RMSNorm, split
+// image and its scale (the partials, image and scales hold the grid's rows only).
+// HBM / L2 bound: reads (z + 1) and writes 2 x 4 bytes per value.
 template <bool EMBED>
 __global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, const float* part, int z,
                                                            const uint16_t* gamma, int row0) {
   __shared__ float s_red[4];
   const int row = row0 + (int)blockIdx.x;
+  const long out = blockIdx.x, n = gridDim.x;
   const long H = a.H;
   float* hr = a.h + row * H;
   float u[kRowChunks][8];
@@ -395,11 +404,11 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, 
     } else {
       load_act8<float>(hr, k, u[c]);
       float p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      const float* src = part + (long)row * H + k;
-#pragma unroll 4
+      const float* src = part + out * H + k;
+#pragma unroll 8
       for (int i = 0; i < z; ++i) {
         float v[8];
-        load_act8<float>(src, (long)i * a.S * H, v);
+        load_act8<float>(src, i * n * H, v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[e] += v[e];
       }
@@ -433,9 +442,9 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, 
     if (k >= H) continue;
 #pragma unroll
     for (int e = 0; e < 8; ++e) u[c][e] *= sc;
-    store_split8(a.img + row * H + k, a.img + ((long)a.S + row) * H + k, u[c]);
+    store_split8(a.img + out * H + k, a.img + (n + out) * H + k, u[c]);
   }
-  if (threadIdx.x == 0) a.scale[row] = pow2f(e2);
+  if (threadIdx.x == 0) a.scale[out] = pow2f(e2);
 }
 
 constexpr int kSiluChunks = 8;   // I up to 16384
@@ -444,7 +453,7 @@ constexpr int kSiluChunks = 8;   // I up to 16384
 // split image and scale.
 __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, int z) {
   __shared__ float s_red[4];
-  const int row = blockIdx.x;
+  const long row = blockIdx.x, n = gridDim.x;
   const long I = a.I;
   float u[kSiluChunks][8];
   float mx = 0.f;
@@ -455,7 +464,7 @@ __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, 
     float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
     for (int i = 0; i < z; ++i) {
-      const float* src = a.part + ((long)i * a.S + row) * 2 * I;
+      const float* src = a.part + (i * n + row) * 2 * I;
       float v[8], w[8];
       load_act8<float>(src, k, v);
       load_act8<float>(src + I, k, w);
@@ -479,7 +488,7 @@ __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, 
     if (k >= I) continue;
 #pragma unroll
     for (int e = 0; e < 8; ++e) u[c][e] *= sc;
-    store_split8(a.img + row * I + k, a.img + ((long)a.S + row) * I + k, u[c]);
+    store_split8(a.img + row * I + k, a.img + (n + row) * I + k, u[c]);
   }
   if (threadIdx.x == 0) a.scale[row] = pow2f(e2);
 }
@@ -574,7 +583,7 @@ __global__ __launch_bounds__(kPrepThreads) void prefill_qkv_prep_kernel(const Pr
   const int r0 = tile * kKvTile + (chunk / 4) * 32 + 4 * (chunk % 4);
   const float* src = a.part + (long)(a.Hq + a.Hkv + kvh) * kHD + d;
   float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
+#pragma unroll 4
   for (int p = 0; p < z; ++p) {
     float x[8];
 #pragma unroll
@@ -609,27 +618,36 @@ __global__ __launch_bounds__(kPrepThreads) void prefill_qkv_prep_kernel(const Pr
 
 // ---------------------------------------------------------------- causal attention
 
+constexpr int kProbExp = 9;       // probabilities relative to the running maximum, times 2^9
+constexpr float kMaxLag = 6.f;
+
 // One workgroup: one q head, 4 waves of 16 QT rows each, the K/V tiles of 64
 // rows up to the diagonal.  S^T = K.Q^T and O^T = V^T.P^T, so that a lane's
 // probabilities (one q row, 4 + 4 kv rows per 32) already are the operand of
 // the second product, and the softmax's row factors are one value per lane.  Each
 // product of split operands is three MFMAs (hi.hi + lo.hi + hi.lo; the dropped
-// lo.lo is 2^-22 of a term).  Probabilities are scaled by 2^13 and by the V
+// lo.lo is 2^-22 of a term).  Probabilities are scaled by 2^9 and by the V
 // tile's exponent against the layer's largest, which keeps them in fp16 range
-// and the accumulators in one unit, 2^(vmax - 13); the output's split image
+// and the accumulators in one unit, 2^(vmax - 9); the output's split image
 // takes 2^vmax as its scale (|o| <= the layer's largest |v|).
 //
-// K and V tiles (32 KB each) are single-buffered: the next K tile is requested
-// when the scores are done, the next V tile after the second product, and two
-// workgroups share a CU, each computing while the other waits.
+// Iteration t multiplies K tile t + 1, takes tile t through the softmax and
+// multiplies V tile t; the tiles of the next iteration are loaded meanwhile into
+// the other of two buffers each, at one barrier per tile.  One workgroup per CU
+// (128 KB of tiles); the grid's heavy (late) tiles start first and the light ones
+// fill in.  28 layers of 4001 rows: 208 us each (a lone workgroup's tile 2.55 us, one
+// under load 3.15, of which its MFMAs take 1.3 at the nominal clock), 1024 rows 36
+// us.  Measured slower: single-buffered tiles with two workgroups per CU (258 / 43
+// us), two q heads of 64 rows on 8 waves, which reads the LDS twice as much (213 /
+// 48), one MFMA to three VALU instructions enforced (255 / 44).
 template <int QT>
-__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L, int layer,
+__global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L, int layer,
                                                                    int q_tiles) {
   constexpr int kPlane = kKvTile * kHD * 2;   // bytes of one K or V plane of a tile
   const int lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int c = lane & 15, g = lane >> 4;
-  // heavy (late) tiles first; one kv head's workgroups share an XCD's L2 when Hkv = 8
+  // one kv head's workgroups share an XCD's L2 when Hkv = 8
   const int kvh = (int)blockIdx.x % a.Hkv, rest = (int)blockIdx.x / a.Hkv;
   const int group = a.Hq / a.Hkv;
   const int head = kvh * group + rest % group;
@@ -644,8 +662,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
   // K tile: 64 rows of 16 chunks, 4 rows per load, chunk c of row r at
   // c ^ (r % 8); V tile: 128 rows (dims) of 8 chunks, 8 rows per load.  Wave w
   // loads rows [16 w, 16 w + 16) of both K planes and dims [32 w, 32 w + 32) of V.
-  auto issue_k = [&](int t) {
-    char* st = lds_stage<0, 2 * kPlane>();
+  auto issue_k = [&](auto B, int t) {
+    char* st = lds_stage<decltype(B)::value, 2 * kPlane>();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * w + 4 * i + (lane >> 4);
@@ -655,8 +673,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
       load_lds16(src + kplane, st + kPlane + (16 * w + 4 * i) * 256);
     }
   };
-  auto issue_v = [&](int t) {
-    char* st = lds_stage<1, 2 * kPlane>();
+  auto issue_v = [&](auto B, int t) {
+    char* st = lds_stage<2 + decltype(B)::value, 2 * kPlane>();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 32 * w + 8 * i + (lane >> 3);
@@ -666,9 +684,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
       load_lds16(src + vplane, st + kPlane + (32 * w + 8 * i) * 128);
     }
   };
-  issue_k(0);
-  issue_v(0);
-
+  const std::integral_constant<int, 0> b0;
+  const std::integral_constant<int, 1> b1;
   // Q operand: column c = row q0 + 16 i + c, k 8 g .. 8 g + 7 of each 32 dims
   h8 qh[QT][4], ql[QT][4];
   const long qplane = (long)a.Hq * a.S * kHD;
@@ -681,10 +698,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
       ql[i][ks] = *reinterpret_cast<const h8*>(src + qplane + 32 * ks);
     }
   }
-  const int emax = a.vmax[layer];
   // log2 units: scale * log2(e) * 2^(q exponent + k exponent)
   const float fac = a.attn_scale * 1.44269504088896340736f * pow2f(head_exp(L.q_norm)) * pow2f(head_exp(L.k_norm));
+  const int emax = ld_scalar(a.vmax + layer);
   if (blockIdx.x == 0 && threadIdx.x == 0) a.o_scale[0] = pow2f(emax);
+  issue_k(b0, 0);
+  issue_v(b0, 0);
+  if (nt > 1) issue_k(b1, 1);
 
   f32x4 o[QT][8];
   float m[QT], l[QT];
@@ -706,86 +726,157 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
     bv[ks] = c * 128 + (((4 * ks + g) ^ (c & 7)) << 4);
     asm("" : "+v"(bv[ks]));
   }
-
-#pragma unroll 1
-  for (int t = 0; t < nt; ++t) {
-    wait_barrier<8>();   // K tile t (V tile t may be in flight)
-    const int ve = ld_scalar(a.vexp + kvh * tiles + t);
-    const char* sk = lds_stage<0, 2 * kPlane>();
-    f32x4 s[QT][4];
+  // (MFMAs of one product over all accumulators before the next product: three
+  // in a row on one accumulator would wait for each other's result)
+  auto scores = [&](auto B, f32x4 (&s)[QT][4]) {
+    const char* sk = lds_stage<decltype(B)::value, 2 * kPlane>();
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < 4; ++n)
 #pragma unroll
       for (int i = 0; i < QT; ++i) s[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const h8 kh = *reinterpret_cast<const h8*>(sk + bk[ks] + n * 16 * 256);
-        const h8 kl = *reinterpret_cast<const h8*>(sk + bk[ks] + kPlane + n * 16 * 256);
+    for (int ks = 0; ks < 4; ++ks) {
+      h8 kh[4], kl[4];
 #pragma unroll
-        for (int i = 0; i < QT; ++i) {
-          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[i][ks], s[i][n], 0, 0, 0);
-          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[i][ks], s[i][n], 0, 0, 0);
-          s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[i][ks], s[i][n], 0, 0, 0);
-        }
+      for (int n = 0; n < 4; ++n) {
+        kh[n] = *reinterpret_cast<const h8*>(sk + bk[ks] + n * 16 * 256);
+        kl[n] = *reinterpret_cast<const h8*>(sk + bk[ks] + kPlane + n * 16 * 256);
       }
-    }
-    wait_barrier<8>();   // every wave is done with K tile t (this wave's V loads stay in flight)
-    issue_k(min(t + 1, nt - 1));
-
-    const float cv = ve - emax + 13 > -126 ? pow2f(ve - emax + 13) : 0.f;
-    const bool diag = t * kKvTile + kKvTile - 1 > q0;
-    h8 ph[QT][2], pl[QT][2];
-#pragma unroll
-    for (int i = 0; i < QT; ++i) {
-      const int lim = q0 + 16 * i + c - t * kKvTile - 4 * g;   // kv 16 n + 4 g + j is visible up to lim
-      float mx = -INFINITY;
 #pragma unroll
       for (int n = 0; n < 4; ++n)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float v = s[i][n][j] * fac;
-          if (diag && 16 * n + j > lim) v = -INFINITY;
-          s[i][n][j] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mn = fmaxf(m[i], mx);
-      const float al = __builtin_amdgcn_exp2f(m[i] - mn);
-      m[i] = mn;
+        for (int i = 0; i < QT; ++i) s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[n], qh[i][ks], s[i][n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int i = 0; i < QT; ++i) s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[n], qh[i][ks], s[i][n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int i = 0; i < QT; ++i) s[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[n], ql[i][ks], s[i][n], 0, 0, 0);
+    }
+  };
+  f32x4 sc[2][QT][4];   // scores of tiles t and t + 1, alternating
+  wait_barrier<0>();
+  scores(b0, sc[0]);
+
+  // iteration t (t % 2 = B): softmax of sc[B], V tile t in V buffer B; MORE: scores of
+  // tile t + 1 from K buffer 1 - B
+  auto body = [&](auto B, auto MORE, int t) {
+    constexpr int b = decltype(B)::value;
+    const std::integral_constant<int, 1 - b> nb;
+    // probabilities leave exp2 already times 2^ve (V tiles 2^-60 below the
+    // layer's largest vanish in the output's fp16 image, whatever their factor)
+    const int ve = max(ld_scalar(a.vexp + kvh * tiles + t) - emax + kProbExp, -60);
+    wait_barrier<0>();   // this iteration's tiles; every wave is done with the buffers refilled below
+    if constexpr (decltype(MORE)::value) {
+      if (t + 2 < nt) issue_k(B, t + 2);
+      issue_v(nb, t + 1);
+      scores(nb, sc[1 - b]);
+    }
+    f32x4 (&s)[QT][4] = sc[b];
+    if (t * kKvTile + kKvTile - 1 > q0) {   // the diagonal: kv 16 n + 4 g + j is visible up to lim
+#pragma unroll
+      for (int i = 0; i < QT; ++i) {
+        const int lim = q0 + 16 * i + c - t * kKvTile - 4 * g;
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (16 * n + j > lim) s[i][n][j] = -INFINITY;
+      }
+    }
+    // The running maximum follows only when a row's has grown by more than
+    // kMaxLag (log2): until then probabilities stay below 2^(kProbExp + kMaxLag),
+    // within fp16, and the accumulators need no rescaling.
+    float mx[QT];
+    bool grow = false;
+#pragma unroll
+    for (int i = 0; i < QT; ++i) {
+      float v = s[i][0][0];
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v = fmaxf(v, s[i][n][j]);
+      v = fmaxf(v, __shfl_xor(v, 16));
+      mx[i] = fmaxf(v, __shfl_xor(v, 32)) * fac;
+      grow = grow || mx[i] > m[i] + kMaxLag;
+    }
+    if (__any(grow)) {
+#pragma unroll
+      for (int i = 0; i < QT; ++i) {
+        const float mn = fmaxf(m[i], mx[i]);
+        const float al = __builtin_amdgcn_exp2f(m[i] - mn);
+        m[i] = mn;
+        l[i] *= al;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) o[i][d] *= al;
+      }
+    }
+    h8 ph[QT][2], pl[QT][2];
+#pragma unroll
+    for (int i = 0; i < QT; ++i) {
+      const float sub = (float)ve - m[i];
       float ps = 0.f;
 #pragma unroll
       for (int n = 0; n < 4; ++n)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float p = __builtin_amdgcn_exp2f(s[i][n][j] - mn);
-          ps += p;
-          _Float16 hi, lo;
-          split2(p * cv, hi, lo);
-          ph[i][n / 2][4 * (n & 1) + j] = hi;
-          pl[i][n / 2][4 * (n & 1) + j] = lo;
+        for (int j = 0; j < 4; j += 2) {
+          f32x2 p;
+          p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][n][j], fac, sub));
+          p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i][n][j + 1], fac, sub));
+          ps += p.x;
+          ps += p.y;
+          const h2 hi = __builtin_convertvector(p, h2);
+          const h2 lo = __builtin_convertvector(p - __builtin_convertvector(hi, f32x2), h2);
+          ph[i][n / 2][4 * (n & 1) + j] = hi.x;
+          ph[i][n / 2][4 * (n & 1) + j + 1] = hi.y;
+          pl[i][n / 2][4 * (n & 1) + j] = lo.x;
+          pl[i][n / 2][4 * (n & 1) + j + 1] = lo.y;
         }
-      l[i] = __builtin_fmaf(l[i], al, ps);
-#pragma unroll
-      for (int d = 0; d < 8; ++d) o[i][d] *= al;
+      l[i] = __builtin_fmaf(ps, pow2f(-ve), l[i]);
     }
-    wait_barrier<8>();   // V tile t (K tile t + 1 may be in flight)
-    const char* sv = lds_stage<1, 2 * kPlane>();
+    const char* sv = lds_stage<2 + b, 2 * kPlane>();
 #pragma unroll
-    for (int d = 0; d < 8; ++d)
+    for (int d0 = 0; d0 < 8; d0 += 4)
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const h8 vh = *reinterpret_cast<const h8*>(sv + bv[ks] + d * 16 * 128);
-        const h8 vl = *reinterpret_cast<const h8*>(sv + bv[ks] + kPlane + d * 16 * 128);
+        h8 vh[4], vl[4];
 #pragma unroll
-        for (int i = 0; i < QT; ++i) {
-          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[i][ks], o[i][d], 0, 0, 0);
-          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[i][ks], o[i][d], 0, 0, 0);
-          o[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[i][ks], o[i][d], 0, 0, 0);
+        for (int d = 0; d < 4; ++d) {
+          vh[d] = *reinterpret_cast<const h8*>(sv + bv[ks] + (d0 + d) * 16 * 128);
+          vl[d] = *reinterpret_cast<const h8*>(sv + bv[ks] + kPlane + (d0 + d) * 16 * 128);
         }
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int i = 0; i < QT; ++i)
+            o[i][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[d], ph[i][ks], o[i][d0 + d], 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int i = 0; i < QT; ++i)
+            o[i][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[d], ph[i][ks], o[i][d0 + d], 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int i = 0; i < QT; ++i)
+            o[i][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[d], pl[i][ks], o[i][d0 + d], 0, 0, 0);
       }
-    wait_barrier<8>();   // every wave is done with V tile t
-    issue_v(min(t + 1, nt - 1));
+  };
+  const std::integral_constant<bool, true> more;
+  const std::integral_constant<bool, false> end;
+  int t = 0;
+#pragma unroll 1
+  for (; t + 2 < nt; t += 2) {
+    body(b0, more, t);
+    body(b1, more, t + 1);
+  }
+  if (t + 1 < nt) {
+    body(b0, more, t);
+    body(b1, end, t + 1);
+  } else {
+    body(b0, end, t);
   }
   const long HD = (long)a.Hq * kHD;
 #pragma unroll
@@ -793,7 +884,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
     l[i] += __shfl_xor(l[i], 16);
     l[i] += __shfl_xor(l[i], 32);
     const int row = q0 + 16 * i + c;
-    const float inv = 1.f / (8192.f * l[i]);
+    const float inv = 1.f / ((float)(1 << kProbExp) * l[i]);
     if (row < a.S) {
       uint16_t* dst = a.img + (long)row * HD + (long)head * kHD + 4 * g;
 #pragma unroll
@@ -811,7 +902,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const Prefill
       }
     }
   }
-  __builtin_amdgcn_s_waitcnt(0x0070);   // the last (unused) tiles have landed before the LDS is given back
 }
 
 }  // namespace
@@ -822,13 +912,15 @@ PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I) {
   PrefillPlan p;
   const long qn = (long)(Hq + 2 * Hkv) * kHD, qs = (long)Hq * kHD;
   p.qkv = split_gemm_plan(S, qn, H);
-  p.o_proj = split_gemm_plan(S, H, qs);
-  p.gate_up = split_gemm_plan(S, 2L * I, H);
-  p.down = split_gemm_plan(S, H, I);
-  const long n[4] = {p.qkv.z * qn, (long)p.o_proj.z * H, p.gate_up.z * 2L * I, (long)p.down.z * H};
-  p.part_floats = 0;
-  for (long x : n)
-    if (x * S > p.part_floats) p.part_floats = x * S;
+  p.part_floats = p.qkv.z * qn * S;
+  for (int l = 0; l < 2; ++l) {
+    const long M = l ? 1 : S;
+    p.o_proj[l] = split_gemm_plan(M, H, qs);
+    p.gate_up[l] = split_gemm_plan(M, 2L * I, H);
+    p.down[l] = split_gemm_plan(M, H, I);
+    for (long x : {(long)p.o_proj[l].z * H, p.gate_up[l].z * 2L * I, (long)p.down[l].z * H})
+      if (x * M > p.part_floats) p.part_floats = x * M;
+  }
   return p;
 }
 
@@ -839,48 +931,53 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
   const long rot = (long)a.S * (kHD / 2), init = rot > a.layers_n ? rot : a.layers_n;
   hipLaunchKernelGGL(prefill_init_kernel, dim3((unsigned)((init + 255) / 256)), dim3(256), 0, s, a);
   if ((st = qd_host::launch_status("prefill_init_kernel"))) return st;
-  auto gemm = [&](const uint16_t* W, const float* scale, int scale_stride, int N, int K, const GemmPlan& g) {
+  // M rows of the image, whose planes lie `plane` values apart
+  auto gemm = [&](const uint16_t* img, long plane, const uint16_t* W, const float* scale, int scale_stride, int M, int N,
+                  int K, const GemmPlan& g) {
     SplitGemmArgs x;
-    x.hi = a.img; x.lo = a.img + (long)a.S * K; x.scale = scale; x.scale_stride = scale_stride; x.W = W; x.y = a.part;
-    x.M = a.S; x.N = N; x.K = K;
+    x.hi = img; x.lo = img + plane; x.scale = scale; x.scale_stride = scale_stride; x.W = W; x.y = a.part;
+    x.M = M; x.N = N; x.K = K;
     return split_gemm_launch(x, g, s);
+  };
+  auto rows = [&](int M, int z, const uint16_t* gamma) {   // the last M rows
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((unsigned)M), dim3(256), 0, s, a, a.part, z, gamma, a.S - M);
+    return qd_host::launch_status("prefill_rows_kernel");
   };
   constexpr int kPrepItems = kPrepThreads / 16;
   const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + kPrepItems - 1) / kPrepItems);
-  // 128 q rows per workgroup once that still gives every CU two workgroups
-  const bool wide = (long)((a.S + 127) / 128) * a.Hq >= 2L * qd_host::cu_count();
-  const int q_tiles = wide ? (a.S + 127) / 128 : (a.S + 63) / 64;
+  // 128 q rows per workgroup where that still gives two rounds of them, which
+  // even out; else 64 (1024 rows: 256 workgroups instead of 128)
+  const int q_rows = (long)((a.S + 127) / 128) * a.Hq >= 2L * qd_host::cu_count() ? 128 : 64;
+  const int q_tiles = (a.S + q_rows - 1) / q_rows;
   for (int li = 0; li < a.layers_n; ++li) {
     const PrefillLayer& L = layers[li];
-    if (li == 0)
+    if (li == 0) {
       hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((unsigned)a.S), dim3(256), 0, s, a, nullptr, 0, L.input_norm, 0);
-    else
-      hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((unsigned)a.S), dim3(256), 0, s, a, a.part, p.down.z,
-                         L.input_norm, 0);
-    if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
-    if ((st = gemm(L.qkv, a.scale, 1, qn, a.H, p.qkv))) return st;
-    hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)),
-                       dim3(kPrepThreads), 0, s, a, L,
-                       p.qkv.z, qk_groups, li);
+      if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
+    } else if ((st = rows(a.S, p.down[0].z, L.input_norm))) {
+      return st;
+    }
+    if ((st = gemm(a.img, (long)a.S * a.H, L.qkv, a.scale, 1, a.S, qn, a.H, p.qkv))) return st;
+    hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)), dim3(kPrepThreads), 0, s, a,
+                       L, p.qkv.z, qk_groups, li);
     if ((st = qd_host::launch_status("prefill_qkv_prep_kernel"))) return st;
-    if (wide)
-      hipLaunchKernelGGL((prefill_attention_kernel<2>), dim3((unsigned)(q_tiles * a.Hq)), dim3(256), 0, s, a, L, li,
-                         q_tiles);
+    // the last layer's K/V rows are written: past them only the last row is used
+    const int last = li + 1 == a.layers_n, M = last ? 1 : a.S;
+    const unsigned groups = (unsigned)a.Hq * (last ? 1u : (unsigned)q_tiles);   // last: its final tile
+    if (q_rows == 128)
+      hipLaunchKernelGGL((prefill_attention_kernel<2>), dim3(groups), dim3(256), 0, s, a, L, li, q_tiles);
     else
-      hipLaunchKernelGGL((prefill_attention_kernel<1>), dim3((unsigned)(q_tiles * a.Hq)), dim3(256), 0, s, a, L, li,
-                         q_tiles);
+      hipLaunchKernelGGL((prefill_attention_kernel<1>), dim3(groups), dim3(256), 0, s, a, L, li, q_tiles);
     if ((st = qd_host::launch_status("prefill_attention_kernel"))) return st;
-    if ((st = gemm(L.o_proj, a.o_scale, 0, a.H, qs, p.o_proj))) return st;
-    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((unsigned)a.S), dim3(256), 0, s, a, a.part, p.o_proj.z,
-                       L.post_norm, 0);
-    if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
-    if ((st = gemm(L.gate_up, a.scale, 1, 2 * a.I, a.H, p.gate_up))) return st;
-    hipLaunchKernelGGL(prefill_silu_kernel, dim3((unsigned)a.S), dim3(256), 0, s, a, p.gate_up.z);
+    if ((st = gemm(a.img + (long)(a.S - M) * qs, (long)a.S * qs, L.o_proj, a.o_scale, 0, M, a.H, qs, p.o_proj[last])))
+      return st;
+    if ((st = rows(M, p.o_proj[last].z, L.post_norm))) return st;
+    if ((st = gemm(a.img, (long)M * a.H, L.gate_up, a.scale, 1, M, 2 * a.I, a.H, p.gate_up[last]))) return st;
+    hipLaunchKernelGGL(prefill_silu_kernel, dim3((unsigned)M), dim3(256), 0, s, a, p.gate_up[last].z);
     if ((st = qd_host::launch_status("prefill_silu_kernel"))) return st;
-    if ((st = gemm(L.down, a.scale, 1, a.H, a.I, p.down))) return st;
+    if ((st = gemm(a.img, (long)M * a.I, L.down, a.scale, 1, M, a.H, a.I, p.down[last]))) return st;
   }
-  hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3(1), dim3(256), 0, s, a, a.part, p.down.z, nullptr, a.S - 1);
-  return qd_host::launch_status("prefill_rows_kernel");
+  return rows(1, p.down[1].z, nullptr);
 }
 
 }  // namespace qd
