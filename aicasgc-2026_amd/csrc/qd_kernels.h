@@ -325,7 +325,8 @@ int decode_persistent_check_device(char* why, size_t why_len);
 
 // y[z][M][N] = scale[m * scale_stride] * (hi + lo)[M][K] . W[N][K]^T over K
 // range z of the plan (fp16 operands, fp32 accumulation).  N % 4 == 0, K a
-// multiple of the plan's tile depth times z, operands below 4 GB each.
+// multiple of the plan's tile depth and at least z times it, operands below 4 GB
+// each.
 struct SplitGemmArgs {
   const uint16_t* hi = nullptr;   // fp16 [M][K]
   const uint16_t* lo = nullptr;   // fp16 [M][K]

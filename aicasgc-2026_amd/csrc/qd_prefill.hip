@@ -145,11 +145,12 @@ __device__ __forceinline__ char* lds_stage() {
 
 // ---------------------------------------------------------------- split GEMM
 
-// y[z][m][n] = scale[m] * sum over the z-th K range of W[n][k] (hi + lo)[m][k].
+// y[z][m][n] = scale[m] * sum over the z-th K range (K / BK blocks, divided as
+// evenly as they go) of W[n][k] (hi + lo)[m][k].
 //
 // Tile BM x BN, BK of K per stage (hi, lo and W rows), NS stages filled by
 // asynchronous global-to-LDS loads NS - 1 steps ahead.  16-byte chunk c of row
-// r sits at c ^ (r % 8) (rows of 128 bytes; c ^ (r / 2 % 4) for 64), so that
+// r sits at c ^ (r % 8) (rows of 128 or 256 bytes; c ^ (r / 2 % 4) for 64), so that
 // the 16 rows a fragment read touches spread over all banks; the permutation is
 // applied to the source address, since the load's LDS side is contiguous.  W is
 // the MFMA A operand, so a lane holds four consecutive outputs of one row.
@@ -161,27 +162,39 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
   constexpr int TM = BM / WM, TN = BN / WN;
   constexpr int CH = BK / 8;
   constexpr int RPI = kWave / CH;                       // rows per load
-  constexpr int LA = BM / RPI / NW, LW = BN / RPI / NW;  // loads per wave and stage
+  constexpr int GA = BM / RPI, GW = BN / RPI;           // loads per stage: of one plane, of W
+  constexpr int LA = (GA + NW - 1) / NW, LW = (GW + NW - 1) / NW;   // and wave
   constexpr int LOADS = 2 * LA + LW;
   constexpr int PA = 2 * BM * BK, STAGE = 2 * PA + 2 * BN * BK;   // bytes
-  static_assert(LA >= 1 && LW >= 1 && (CH == 8 || CH == 4) && LOADS * (NS - 1) < 64 && NS == 3, "tile shape");
+  static_assert(BM % RPI == 0 && BN % RPI == 0 && TM % 16 == 0 && TN % 16 == 0 && (CH == 16 || CH == 8 || CH == 4) &&
+                    LOADS * (NS - 1) < 64 && NS == 3, "tile shape");
   const int lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int tiles_m = (a.M + BM - 1) / BM;
   const int q = (int)gridDim.x >> 3, r = (int)gridDim.x & 7, xcd = (int)blockIdx.x & 7, loc = (int)blockIdx.x >> 3;
   const int t = xcd * q + min(xcd, r) + loc;
   const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
-  const int kz = a.K / (int)gridDim.y, nk = kz / BK;
-  const long kbase = (long)blockIdx.y * kz;
+  const int kblocks = a.K / BK, kfirst = kblocks * (int)blockIdx.y / (int)gridDim.y;
+  const int nk = kblocks * ((int)blockIdx.y + 1) / (int)gridDim.y - kfirst;
+  const long kbase = (long)kfirst * BK;
   const int lr = lane / CH, lc = lane % CH;
-  const int sc = lc ^ (CH == 8 ? (lr & 7) : ((lr >> 1) & 3));
+  // where the waves do not divide the loads, the last load is issued more than
+  // once (same data, same place), so that every wave counts the same number
   unsigned offA[LA], offW[LW];
+  int dstA[LA], dstW[LW];
+  auto swz = [](int r) { return CH == 4 ? ((r >> 1) & 3) : (r & 7); };
 #pragma unroll
-  for (int i = 0; i < LA; ++i)
-    offA[i] = ((unsigned)min(m0 + (i * NW + w) * RPI + lr, a.M - 1) * (unsigned)a.K + sc * 8) * 2u;
+  for (int i = 0; i < LA; ++i) {
+    const int g = min(i * NW + w, GA - 1), r = g * RPI + lr;
+    dstA[i] = g * 1024;
+    offA[i] = ((unsigned)min(m0 + r, a.M - 1) * (unsigned)a.K + (lc ^ swz(r)) * 8) * 2u;
+  }
 #pragma unroll
-  for (int i = 0; i < LW; ++i)
-    offW[i] = ((unsigned)min(n0 + (i * NW + w) * RPI + lr, a.N - 1) * (unsigned)a.K + sc * 8) * 2u;
+  for (int i = 0; i < LW; ++i) {
+    const int g = min(i * NW + w, GW - 1), r = g * RPI + lr;
+    dstW[i] = 2 * PA + g * 1024;
+    offW[i] = ((unsigned)min(n0 + r, a.N - 1) * (unsigned)a.K + (lc ^ swz(r)) * 8) * 2u;
+  }
   const char* Ah = reinterpret_cast<const char*>(a.hi + kbase);
   const char* Al = reinterpret_cast<const char*>(a.lo + kbase);
   const char* Wp = reinterpret_cast<const char*>(a.W + kbase);
@@ -190,11 +203,11 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
     const long ko = (long)k * BK * 2;
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
-      load_lds16(Ah + ko + offA[i], st + (i * NW + w) * 1024);
-      load_lds16(Al + ko + offA[i], st + PA + (i * NW + w) * 1024);
+      load_lds16(Ah + ko + offA[i], st + dstA[i]);
+      load_lds16(Al + ko + offA[i], st + PA + dstA[i]);
     }
 #pragma unroll
-    for (int i = 0; i < LW; ++i) load_lds16(Wp + ko + offW[i], st + 2 * PA + (i * NW + w) * 1024);
+    for (int i = 0; i < LW; ++i) load_lds16(Wp + ko + offW[i], st + dstW[i]);
   };
   f32x4 acc[TM / 16][TN / 16];
 #pragma unroll
@@ -203,7 +216,7 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
     for (int j = 0; j < TN / 16; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int wm = w / WN, wn = w % WN;
   const int fr = lane & 15, fg = lane >> 4;
-  const int fs = CH == 8 ? (fr & 7) : ((fr >> 1) & 3);
+  const int fs = swz(fr);
   // byte offsets of this lane's fragments, opaque so that every fragment
   // address stays one base plus a constant
   unsigned bA[BK / 32], bW[BK / 32];
@@ -287,20 +300,27 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
 
 namespace {
 
-// Tile shapes, 8 waves each (4 along m, 2 along n: a wave's W rows are read from
-// LDS once for both planes, so wide wave tiles read least), and their cost: a
-// workgroup's microseconds per 1024 of K with every CU busy, beside ~3 us of
-// ramp, and how many share a CU.  Measured at the 2B shapes (MFMA rate):
-// 344 us (1169 TFLOP/s) at 4001 x 12288 x 2048 on 256 x 256, 177 us (1140) at
-// 4001 x 2048 x 6144 on 128 x 256, 35 us (975) at 1024 x 4096 x 2048 on
-// 128 x 128, where four waves of 64 x 64 took 40.
+// Tile shapes (8 waves; wide wave tiles read the LDS least, since a wave reads its
+// W rows once for both planes) and their cost: `ramp` us per workgroup and `us`
+// per 1024 of K with every CU busy, `idle` of that on an almost idle chip, and
+// the TB/s its loads and stores reach.  Fitted to every shape and K split at
+// 1 .. 4001 rows of the four 2B products (W cold, one workgroup per CU; 4 to 8 %
+// rms, the chosen pair 2.8 % behind the best measured one on average).  The widths
+// of 192 and the rows below 64 are there for the rounds: 1024 x 12288 x 2048 takes
+// 192 workgroups of 256 x 256 (98 us) or 256 of 256 x 192 (88), 512 rows 58 or 53
+// us; 1300 x 12288 x 2048 148 us on 128 x 128, 134 on 192 x 192.  16 rows of 12288
+// x 2048 take 14.1 us on 64-row tiles, 11.6 on 32 x 128 with 128 of K per stage.
 struct GemmTile {
-  int bm, bn, bk, per_cu;
-  float us;
+  int bm, bn, bk;
+  float ramp, us, idle, tbs;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {256, 256, 32, 1, 57.f}, {128, 256, 32, 1, 29.f},  {128, 128, 64, 1, 16.f},
-    {64, 128, 64, 1, 11.f}, {64, 64, 64, 2, 12.f},
+    {256, 256, 32, 12.0f, 46.6f, 0.71f, 3.75f}, {256, 192, 32, 9.2f, 37.8f, 0.76f, 3.69f},
+    {192, 192, 32, 7.3f, 31.6f, 0.80f, 3.71f},  {128, 256, 32, 7.5f, 26.2f, 0.75f, 3.45f},
+    {128, 128, 64, 4.2f, 14.4f, 0.77f, 3.59f},  {64, 256, 64, 4.3f, 15.9f, 0.77f, 4.71f},
+    {64, 192, 64, 3.5f, 12.6f, 0.82f, 5.02f},   {64, 128, 64, 2.4f, 9.7f, 0.86f, 4.48f},
+    {64, 64, 128, 2.1f, 6.1f, 0.95f, 4.15f},    {32, 128, 128, 2.4f, 7.3f, 0.82f, 5.36f},
+    {32, 64, 128, 2.0f, 4.7f, 0.92f, 5.20f},    {16, 128, 128, 2.0f, 5.5f, 0.99f, 5.27f},
 };
 
 template <int BM, int BN, int BK, int WM, int WN>
@@ -312,23 +332,27 @@ int launch_gemm(const SplitGemmArgs& a, int z, hipStream_t s) {
 
 }  // namespace
 
-// The tile shape and K split with the least estimated time: rounds of
-// workgroups over the CUs, each costing its K range's tile time plus a fixed
-// ~3 us, plus the partial planes written and read again (~4 TB/s).
+// The tile shape and K split with the least estimated time: rounds of workgroups
+// over the CUs or the bytes they move, whichever is longer (summed in the fourth
+// power, as the two overlap), plus the partial planes read again (~4 TB/s).
 GemmPlan split_gemm_plan(long M, long N, long K) {
   GemmPlan best{-1, 1};
   float best_us = 0.f;
   const int cus = qd_host::cu_count();
   for (int c = 0; c < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++c) {
     const GemmTile& g = kGemmTiles[c];
-    for (int z = 1; z <= kPrefillMaxSplit; z *= 2) {
-      if (K % ((long)g.bk * z) != 0) break;
+    if (K % g.bk != 0) continue;
+    for (int z : {1, 2, 3, 4, 6, 8, 12, kPrefillMaxSplit}) {
+      if (K / g.bk < z) break;
       const long wgs = ((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn) * z;
-      const long rounds = (wgs + (long)cus * g.per_cu - 1) / ((long)cus * g.per_cu);
-      // a grid that leaves CUs idle runs each workgroup faster (64 / 192 of 256 CUs: 0.72 / 0.82)
-      const float fill = (float)wgs / (float)(rounds * cus * g.per_cu);
-      const float us = (float)rounds * (3.f + (0.7f + 0.3f * fill * fill) * g.us * (float)(K / z) / 1024.f) +
-                       8.f * (float)z * (float)M * (float)N / 4e6f;
+      const long rounds = (wgs + cus - 1) / cus;
+      const float fill = (float)wgs / (float)(rounds * cus);
+      const float compute =
+          (float)rounds * (g.ramp + (g.idle + (1.f - g.idle) * fill * fill) * g.us * (float)K / (float)z / 1024.f);
+      const float planes = 4.f * (float)z * (float)M * (float)N;
+      const float memory = 2.f + (2.f * (float)N * (float)K + 4.f * (float)M * (float)K + planes) / (g.tbs * 1e6f);
+      const float c2 = compute * compute, m2 = memory * memory;
+      const float us = sqrtf(sqrtf(c2 * c2 + m2 * m2)) + planes / 4e6f;
       if (best.tile < 0 || us < best_us) {
         best = GemmPlan{c, z};
         best_us = us;
@@ -339,16 +363,24 @@ GemmPlan split_gemm_plan(long M, long N, long K) {
 }
 
 int split_gemm_launch(const SplitGemmArgs& a, const GemmPlan& p, hipStream_t s) {
-  if (a.M < 1 || a.N < 4 || a.N % 4 != 0 || p.tile < 0 || p.z < 1 || a.K % ((long)kGemmTiles[p.tile].bk * p.z) != 0)
+  if (a.M < 1 || a.N < 4 || a.N % 4 != 0 || p.tile < 0 || p.z < 1 || a.K % kGemmTiles[p.tile].bk != 0 ||
+      a.K / kGemmTiles[p.tile].bk < p.z)
     return QD_ERR_SHAPE;
   // 32-bit byte offsets into the operands
   if ((size_t)a.M * a.K * 2 >> 32 || (size_t)a.N * a.K * 2 >> 32) return QD_ERR_SHAPE;
   switch (p.tile) {
     case 0: return launch_gemm<256, 256, 32, 4, 2>(a, p.z, s);
-    case 1: return launch_gemm<128, 256, 32, 4, 2>(a, p.z, s);
-    case 2: return launch_gemm<128, 128, 64, 4, 2>(a, p.z, s);
-    case 3: return launch_gemm<64, 128, 64, 4, 2>(a, p.z, s);
-    default: return launch_gemm<64, 64, 64, 4, 2>(a, p.z, s);
+    case 1: return launch_gemm<256, 192, 32, 4, 2>(a, p.z, s);
+    case 2: return launch_gemm<192, 192, 32, 4, 2>(a, p.z, s);
+    case 3: return launch_gemm<128, 256, 32, 4, 2>(a, p.z, s);
+    case 4: return launch_gemm<128, 128, 64, 4, 2>(a, p.z, s);
+    case 5: return launch_gemm<64, 256, 64, 4, 2>(a, p.z, s);
+    case 6: return launch_gemm<64, 192, 64, 4, 2>(a, p.z, s);
+    case 7: return launch_gemm<64, 128, 64, 4, 2>(a, p.z, s);
+    case 8: return launch_gemm<64, 64, 128, 4, 2>(a, p.z, s);
+    case 9: return launch_gemm<32, 128, 128, 2, 4>(a, p.z, s);
+    case 10: return launch_gemm<32, 64, 128, 2, 4>(a, p.z, s);
+    default: return launch_gemm<16, 128, 128, 1, 8>(a, p.z, s);
   }
 }
 

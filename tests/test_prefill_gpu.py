@@ -69,6 +69,13 @@ def test_prefill_text_lengths(cuda, n):
     _run(f"text {n}", MODEL, None, n)
 
 
+@pytest.mark.parametrize("n", [15, 33, 49, 193, 300, 700, 1300])
+def test_prefill_tile_shapes(cuda, n):
+    """Lengths at which the four products take the 16-, 32- and 64-row tiles, the
+    192-wide ones and K ranges of unequal length."""
+    _run(f"tiles {n}", MODEL, None, n)
+
+
 @pytest.mark.parametrize("grid,n_text", [((3, 5), 1), ((7, 9), 2), ((24, 32), 330), ((40, 44), 351)])
 def test_prefill_multimodal(cuda, grid, n_text):
     _run(f"grid {grid} text {n_text}", MODEL, grid, n_text)
