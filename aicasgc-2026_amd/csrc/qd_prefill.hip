@@ -977,9 +977,11 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
   };
   constexpr int kPrepItems = kPrepThreads / 16;
   const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + kPrepItems - 1) / kPrepItems);
-  // 128 q rows per workgroup where that still gives two rounds of them, which
-  // even out; else 64 (1024 rows: 256 workgroups instead of 128)
-  const int q_rows = (long)((a.S + 127) / 128) * a.Hq >= 2L * qd_host::cu_count() ? 128 : 64;
+  // 128 q rows per workgroup read the LDS half as often, 64 give twice the
+  // workgroups; they meet at 1.25 workgroups of 128 rows per CU (28 layers of 2B, 64 /
+  // 128 rows: 1800 rows 13.25 / 13.74 ms, 2432 17.50 / 17.64, 2560 18.18 / 18.14, 3000
+  // 22.5 / 22.0, 3800 27.8 / 26.6)
+  const int q_rows = (long)((a.S + 127) / 128) * a.Hq * 4 >= 5L * qd_host::cu_count() ? 128 : 64;
   const int q_tiles = (a.S + q_rows - 1) / q_rows;
   for (int li = 0; li < a.layers_n; ++li) {
     const PrefillLayer& L = layers[li];

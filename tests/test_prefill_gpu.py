@@ -76,6 +76,13 @@ def test_prefill_tile_shapes(cuda, n):
     _run(f"tiles {n}", MODEL, None, n)
 
 
+@pytest.mark.parametrize("n", [2432, 2433, 2560])
+def test_prefill_attention_tile_rows(cuda, n):
+    """Both sides of the step from 64 to 128 q rows per attention workgroup (16
+    heads, 256 CUs), and an even multiple of the larger tile."""
+    _run(f"q tiles {n}", MODEL, None, n, layers=1)
+
+
 @pytest.mark.parametrize("grid,n_text", [((3, 5), 1), ((7, 9), 2), ((24, 32), 330), ((40, 44), 351)])
 def test_prefill_multimodal(cuda, grid, n_text):
     _run(f"grid {grid} text {n_text}", MODEL, grid, n_text)
