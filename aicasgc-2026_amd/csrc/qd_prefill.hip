@@ -730,8 +730,11 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
       ql[i][ks] = *reinterpret_cast<const h8*>(src + qplane + 32 * ks);
     }
   }
-  // log2 units: scale * log2(e) * 2^(q exponent + k exponent)
-  const float fac = a.attn_scale * 1.44269504088896340736f * pow2f(head_exp(L.q_norm)) * pow2f(head_exp(L.k_norm));
+  // log2 units: scale * log2(e) * 2^(q exponent + k exponent).  Both head norms
+  // all zero would underflow it to 0 (their scores are 0) and the masked -inf
+  // scores times that to NaN; other fp16 weights keep it above 2^-76.
+  const float fac = fmaxf(
+      a.attn_scale * 1.44269504088896340736f * pow2f(head_exp(L.q_norm)) * pow2f(head_exp(L.k_norm)), 0x1p-120f);
   const int emax = ld_scalar(a.vmax + layer);
   if (blockIdx.x == 0 && threadIdx.x == 0) a.o_scale[0] = pow2f(emax);
   issue_k(b0, 0);

@@ -41,7 +41,7 @@ def _check(w, prompt, eng, token):
     assert float(logits.max() - logits[token]) <= 1e-4 * float(logits.abs().max())
 
 
-def _run(case, shape_kw, grid, n_text, layers=2, scale=None):
+def _run(case, shape_kw, grid, n_text, layers=2, scale=None, weights=None):
     from qwen3vl_hip import _lib, synthetic as syn
     from qwen3vl_hip.config import Qwen3VLTextShape
     from qwen3vl_hip.engine import DecodeEngine
@@ -51,6 +51,8 @@ def _run(case, shape_kw, grid, n_text, layers=2, scale=None):
     print(f"case prefill {case}", flush=True)
     shape = Qwen3VLTextShape(num_layers=layers, **shape_kw)
     w = syn.model_weights(11, shape)
+    if weights is not None:
+        weights(w)
     p = syn.multimodal_prompt(11, *((1, *grid) if grid else (0, 0, 0)), n_text, shape=shape)
     if scale is not None:
         p = dataclasses.replace(p, vision_embeds=p.vision_embeds.float() * scale(p.vision_embeds.shape[0])[:, None])
@@ -98,6 +100,13 @@ def test_prefill_rows_of_very_different_magnitude(cuda):
     """fp32 embedding rows from 1e-4 to 1e4 of the usual size, in one prompt."""
     _run("scaled rows", MODEL, (8, 11), 9,
          scale=lambda n: 10.0 ** (torch.arange(n) % 9 - 4).float())
+
+
+@pytest.mark.parametrize("n", [5, 70])
+def test_prefill_zero_head_norms(cuda, n):
+    """q and k norm weights of zero: all scores equal, attention the causal mean."""
+    _run(f"zero head norms {n}", SMALL, None, n,
+         weights=lambda w: [t.zero_() for lw in w.layers for t in (lw.q_norm_weight, lw.k_norm_weight)])
 
 
 def test_prefill_forms_outside_the_native_route(cuda):
