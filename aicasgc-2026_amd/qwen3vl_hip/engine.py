@@ -34,15 +34,18 @@ def rope_inv_freq(shape: Qwen3VLTextShape = QWEN3VL_2B) -> torch.Tensor:
 
 
 def _host_ints(x, n: int):
-    """The n values of a list, a tuple, a number or a CPU tensor as a ctypes
-    int64 array, or None for anything else (a device tensor stays there)."""
+    """The n values of a flat list, tuple or CPU tensor, or a number, as a
+    ctypes int64 array, or None for anything else (a device tensor stays there,
+    nested and multi-dimensional forms broadcast as torch has it)."""
     if torch.is_tensor(x):
-        if x.is_cuda:
+        if x.is_cuda or x.ndim != 1:
             return None
-        x = x.reshape(-1).tolist()
+        x = x.tolist()
     elif not isinstance(x, (list, tuple)):
         x = [x]
-    return (ctypes.c_int64 * n)(*(int(v) for v in x)) if len(x) == n else None
+    if len(x) != n or any(isinstance(v, (list, tuple)) or getattr(v, "shape", ()) != () for v in x):
+        return None
+    return (ctypes.c_int64 * n)(*(int(v) for v in x))
 
 
 class _CapturedSteps:

@@ -94,7 +94,7 @@ def test_full_model_config3_first_64_tokens(cuda, config3_weights, step_mode):
     assert toks == ref
 
 
-@pytest.mark.parametrize("form", ["lists", "cpu tensors", "device tensors", "one for all"])
+@pytest.mark.parametrize("form", ["lists", "cpu tensors", "device tensors", "one for all", "column"])
 def test_batch_state_forms(cuda, form):
     """The step state set from host values in one launch, from device tensors, or broadcast."""
     from qwen3vl_hip import synthetic as syn
@@ -106,6 +106,8 @@ def test_batch_state_forms(cuda, form):
     want = [v * (3 // len(v)) for v in vals]
     if "tensors" in form:
         vals = tuple(torch.tensor(v, device=cuda if form.startswith("device") else "cpu") for v in vals)
+    if form == "column":   # rope positions [batch, 1]
+        vals = (vals[0], vals[1], [[p] for p in vals[2]])
     eng.step_counter.fill_(5)
     eng.set_state(*vals)
     assert eng.token.tolist() == want[0] and eng.cache_position.tolist() == want[1]
