@@ -7,7 +7,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -1336,7 +1338,8 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
   QD_REQUIRE(workspace_bytes >= need && aligned(workspace, 256), QD_ERR_WORKSPACE,
              "workspace of %zu bytes, 256-byte aligned (got %zu)", need, workspace_bytes);
   QD_REQUIRE(a16(d->embed) && a16(d->final_norm), QD_ERR_ARG, "weights must be 16-byte aligned");
-  std::vector<qd::PrefillLayer> layers((size_t)d->num_layers);
+  std::unique_ptr<qd::PrefillLayer[]> layers(new (std::nothrow) qd::PrefillLayer[(size_t)d->num_layers]);
+  QD_REQUIRE(layers, QD_ERR_ARG, "no host memory for %d layers", d->num_layers);
   for (int i = 0; i < d->num_layers; ++i) {
     const qd_layer_weights& w = d->layers[i];
     QD_REQUIRE(w.qkv && w.o_proj && w.gate_up && w.down && w.input_norm && w.post_norm && w.q_norm && w.k_norm &&
@@ -1345,10 +1348,10 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
     QD_REQUIRE(a16(w.qkv) && a16(w.o_proj) && a16(w.gate_up) && a16(w.down) && a16(w.input_norm) && a16(w.post_norm) &&
                    aligned(w.k_cache, 8),
                QD_ERR_ARG, "layer %d: weights must be 16-byte aligned, the K cache 8-byte", i);
-    layers[(size_t)i] = qd::PrefillLayer{(const u16*)w.qkv,        (const u16*)w.o_proj,    (const u16*)w.gate_up,
-                                         (const u16*)w.down,       (const u16*)w.input_norm, (const u16*)w.post_norm,
-                                         (const u16*)w.q_norm,     (const u16*)w.k_norm,    (u16*)w.k_cache,
-                                         (u16*)w.v_cache};
+    layers[i] = qd::PrefillLayer{(const u16*)w.qkv,    (const u16*)w.o_proj,     (const u16*)w.gate_up,
+                                 (const u16*)w.down,   (const u16*)w.input_norm, (const u16*)w.post_norm,
+                                 (const u16*)w.q_norm, (const u16*)w.k_norm,     (u16*)w.k_cache,
+                                 (u16*)w.v_cache};
   }
   char* base = reinterpret_cast<char*>(workspace);
   qd::PrefillArgs a;
@@ -1369,7 +1372,7 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
   a.vexp = reinterpret_cast<int*>(base + b.vexp);
   a.vmax = reinterpret_cast<int*>(base + b.vmax);
   a.argmax_count = reinterpret_cast<unsigned*>(base + b.argmax);
-  const int st = qd::prefill_launch(a, layers.data(), plan, S(stream));
+  const int st = qd::prefill_launch(a, layers.get(), plan, S(stream));
   if (st) return st;
   return qd_lm_head_argmax(a.h + (size_t)(rows - 1) * d->hidden, QD_F32, d->final_norm, d->eps, d->embed, d->vocab,
                            d->hidden, nullptr, token_out, base + b.argmax, stream);
