@@ -479,22 +479,28 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const PrefillArgs a, 
   if (threadIdx.x == 0) a.scale[out] = pow2f(e2);
 }
 
-constexpr int kSiluChunks = 8;   // I up to 16384
+constexpr int kMaxI = 16384;
 
 // One row per workgroup: hidden = silu(gate) * up from the gate_up partials,
-// split image and scale.
-__global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, int z) {
-  __shared__ float s_red[4];
+// split image and scale.  A few rows are bound by the chain of plane loads of a
+// thread's chunks, so up to one row per CU takes 1024 threads and, at I = 6144, one
+// chunk per thread; beyond, workgroups of 256 hide it and end more evenly.
+// Measured, 256 / 1024 threads, us: 17 rows 5.8 / 4.5, 37 6.8 / 5.1, 128 6.6 / 5.6,
+// 256 6.8 / 6.1, 300 7.3 / 8.1, 700 10.4 / 12.2, 4001 48.6 (6.1 TB/s) / 59.4.
+template <int NT>
+__global__ __launch_bounds__(NT) void prefill_silu_kernel(const PrefillArgs a, int z) {
+  constexpr int kChunks = kMaxI / (8 * NT);
+  __shared__ float s_red[NT / kWave];
   const long row = blockIdx.x, n = gridDim.x;
   const long I = a.I;
-  float u[kSiluChunks][8];
+  float u[kChunks][8];
   float mx = 0.f;
 #pragma unroll
-  for (int c = 0; c < kSiluChunks; ++c) {
-    const long k = (long)c * 2048 + threadIdx.x * 8;
+  for (int c = 0; c < kChunks; ++c) {
+    const long k = (long)c * 8 * NT + threadIdx.x * 8;
     if (k >= I) continue;
     float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
+#pragma unroll (NT > 256 ? 4 : 2)
     for (int i = 0; i < z; ++i) {
       const float* src = a.part + (i * n + row) * 2 * I;
       float v[8], w[8];
@@ -512,11 +518,11 @@ __global__ __launch_bounds__(256) void prefill_silu_kernel(const PrefillArgs a, 
       mx = fmaxf(mx, fabsf(u[c][e]));
     }
   }
-  const int e2 = split_exp(block_max(mx, s_red, 4));
+  const int e2 = split_exp(block_max(mx, s_red, NT / kWave));
   const float sc = pow2f(-e2);
 #pragma unroll
-  for (int c = 0; c < kSiluChunks; ++c) {
-    const long k = (long)c * 2048 + threadIdx.x * 8;
+  for (int c = 0; c < kChunks; ++c) {
+    const long k = (long)c * 8 * NT + threadIdx.x * 8;
     if (k >= I) continue;
 #pragma unroll
     for (int e = 0; e < 8; ++e) u[c][e] *= sc;
@@ -1010,7 +1016,10 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
       return st;
     if ((st = rows(M, p.o_proj[last].z, L.post_norm))) return st;
     if ((st = gemm(a.img, (long)M * a.H, L.gate_up, a.scale, 1, M, 2 * a.I, a.H, p.gate_up[last]))) return st;
-    hipLaunchKernelGGL(prefill_silu_kernel, dim3((unsigned)M), dim3(256), 0, s, a, p.gate_up[last].z);
+    if (M <= qd_host::cu_count())
+      hipLaunchKernelGGL(prefill_silu_kernel<1024>, dim3((unsigned)M), dim3(1024), 0, s, a, p.gate_up[last].z);
+    else
+      hipLaunchKernelGGL(prefill_silu_kernel<256>, dim3((unsigned)M), dim3(256), 0, s, a, p.gate_up[last].z);
     if ((st = qd_host::launch_status("prefill_silu_kernel"))) return st;
     if ((st = gemm(a.img, (long)M * a.I, L.down, a.scale, 1, M, a.H, a.I, p.down[last]))) return st;
   }

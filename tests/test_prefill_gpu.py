@@ -71,10 +71,11 @@ def test_prefill_text_lengths(cuda, n):
     _run(f"text {n}", MODEL, None, n)
 
 
-@pytest.mark.parametrize("n", [15, 33, 49, 193, 300, 700, 1300])
+@pytest.mark.parametrize("n", [15, 33, 49, 193, 256, 300, 700, 1300])
 def test_prefill_tile_shapes(cuda, n):
     """Lengths at which the four products take the 16-, 32- and 64-row tiles, the
-    192-wide ones and K ranges of unequal length."""
+    192-wide ones and K ranges of unequal length; 256 is the last with 1024 threads
+    per SiLU row on 256 CUs."""
     _run(f"tiles {n}", MODEL, None, n)
 
 
