@@ -1271,7 +1271,7 @@ int qd_batch_gemv(const float* x, long ldx, const void* gamma, float eps, const 
 namespace {
 
 struct PrefillBuffers {
-  size_t h, img, scale, o_scale, part, cs, q_img, k_img, vt_img, vexp, vmax, argmax;
+  size_t h, img, scale, part, cs, q_img, k_img, vt_img, vexp, argmax;
 };
 
 // Workspace of a prefill of S rows, or 0 where the kernels do not apply.
@@ -1299,14 +1299,12 @@ size_t prefill_layout(const qd_model_desc* d, long S_, qd::PrefillPlan* plan, Pr
   b->h = take(4 * (size_t)S_ * H);
   b->img = take(4 * (size_t)S_ * kmax);
   b->scale = take(4 * (size_t)S_);
-  b->o_scale = take(4);
   b->part = take(4 * (size_t)plan->part_floats);
   b->cs = take(8 * (size_t)S_ * 64);
   b->q_img = take(4 * (size_t)S_ * qs);
   b->k_img = take(4 * (size_t)S_ * Hkv * 128);
   b->vt_img = take(4 * (size_t)tiles * 64 * Hkv * 128);
   b->vexp = take(4 * (size_t)tiles * Hkv);
-  b->vmax = take(4 * (size_t)d->num_layers);
   b->argmax = take(argmax_ws_bytes());
   return off;
 }
@@ -1363,14 +1361,12 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
   a.h = reinterpret_cast<float*>(base + b.h);
   a.img = reinterpret_cast<u16*>(base + b.img);
   a.scale = reinterpret_cast<float*>(base + b.scale);
-  a.o_scale = reinterpret_cast<float*>(base + b.o_scale);
   a.part = reinterpret_cast<float*>(base + b.part);
   a.cs = reinterpret_cast<float2*>(base + b.cs);
   a.q_img = reinterpret_cast<u16*>(base + b.q_img);
   a.k_img = reinterpret_cast<u16*>(base + b.k_img);
   a.vt_img = reinterpret_cast<u16*>(base + b.vt_img);
   a.vexp = reinterpret_cast<int*>(base + b.vexp);
-  a.vmax = reinterpret_cast<int*>(base + b.vmax);
   a.argmax_count = reinterpret_cast<unsigned*>(base + b.argmax);
   const int st = qd::prefill_launch(a, layers.get(), plan, S(stream));
   if (st) return st;

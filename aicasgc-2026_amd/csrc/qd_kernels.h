@@ -323,15 +323,14 @@ int decode_persistent_check_device(char* why, size_t why_len);
 
 // ---------------------------------------------------------------- prefill
 
-// y[z][M][N] = scale[m * scale_stride] * (hi + lo)[M][K] . W[N][K]^T over K
+// y[z][M][N] = scale[m] * (hi + lo)[M][K] . W[N][K]^T over K
 // range z of the plan (fp16 operands, fp32 accumulation).  N % 4 == 0, K a
 // multiple of the plan's tile depth and at least z times it, operands below 4 GB
 // each.
 struct SplitGemmArgs {
   const uint16_t* hi = nullptr;   // fp16 [M][K]
   const uint16_t* lo = nullptr;   // fp16 [M][K]
-  const float* scale = nullptr;
-  int scale_stride = 1;           // 1: one scale per row; 0: one for all rows
+  const float* scale = nullptr;   // [M]
   const uint16_t* W = nullptr;    // fp16 [N][K]
   float* y = nullptr;             // fp32 [z][M][N]
   int M = 0, N = 0, K = 0;
@@ -364,14 +363,12 @@ struct PrefillArgs {
   float* h;                       // [S][H] residual stream
   uint16_t* img;                  // split image (hi plane, lo plane) of the next GEMM's input
   float* scale;                   // [S] its row scales
-  float* o_scale;                 // [1] scale of the attention output's image
   float* part;                    // GEMM output planes
   float2* cs;                     // [S][64] cos, sin
   uint16_t* q_img;                // 2 x [Hq][S][128]
   uint16_t* k_img;                // 2 x [Hkv][S][128]
   uint16_t* vt_img;               // 2 x [Hkv][tiles][128][64]
-  int* vexp;                      // [Hkv][tiles] exponents of the V tiles
-  int* vmax;                      // [layers] largest of them
+  int* vexp;                      // [tiles][Hkv] exponents of the V tiles
   unsigned* argmax_count;         // [64] cleared for the lm_head
 };
 struct PrefillPlan {

@@ -44,6 +44,7 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kHD = 128;        // head dim
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kWave * WM * WN) void split_gemm_kernel(const Split
   float scale[TM / 16];
 #pragma unroll
   for (int i = 0; i < TM / 16; ++i)
-    scale[i] = a.scale[(long)min(m0 + wm * TM + 16 * i + fr, a.M - 1) * a.scale_stride];
+    scale[i] = a.scale[min(m0 + wm * TM + 16 * i + fr, a.M - 1)];
   float* y = a.y + (long)blockIdx.y * a.M * a.N;
 #pragma unroll
   for (int i = 0; i < TM / 16; ++i) {
@@ -389,10 +390,9 @@ namespace {
 // ---------------------------------------------------------------- elementwise launches
 
 // cos / sin of every (row, rotary pair), fp32 angles as the decode step's, and
-// the words that must start at zero (exponent maxima, the argmax counter).
+// the argmax counter's zeros.
 __global__ __launch_bounds__(256) void prefill_init_kernel(const PrefillArgs a) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < a.layers_n) a.vmax[i] = -kMaxExp;
   if (i < 64) a.argmax_count[i] = 0u;
   if (i >= (long)a.S * (kHD / 2)) return;
   const int row = (int)(i / (kHD / 2)), j = (int)(i % (kHD / 2));
@@ -548,10 +548,9 @@ constexpr int kPrepThreads = 1024;
 // 16 (e / 4) + 4 g + e % 4.  A thread owns one 16-byte chunk of that image, so 8
 // rows of one dim; all its loads are issued before its first store (32 rows a
 // thread, each stored before the next was loaded: 66 us instead of ~9 for 37
-// rows and 8 planes).  The tile's exponent goes to vexp and, as the layer's
-// maximum, to vmax.
+// rows and 8 planes).  The tile's exponent goes to vexp.
 __global__ __launch_bounds__(kPrepThreads) void prefill_qkv_prep_kernel(const PrefillArgs a, const PrefillLayer L,
-                                                                        int z, int qk_groups, int layer) {
+                                                                        int z, int qk_groups) {
   __shared__ float s_red[kPrepThreads / kWave];
   const long NQ = (long)(a.Hq + 2 * a.Hkv) * kHD;
   if ((int)blockIdx.x < qk_groups) {
@@ -648,38 +647,47 @@ __global__ __launch_bounds__(kPrepThreads) void prefill_qkv_prep_kernel(const Pr
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] *= sc;
   store_split8(dst, dst + plane, v);
-  if (threadIdx.x == 0) {
-    a.vexp[it] = ex;
-    atomicMax(a.vmax + layer, ex);
-  }
+  if (threadIdx.x == 0) a.vexp[(long)tile * a.Hkv + kvh] = ex;
 }
 
 // ---------------------------------------------------------------- causal attention
 
 constexpr int kProbExp = 9;       // probabilities relative to the running maximum, times 2^9
 constexpr float kMaxLag = 6.f;
+constexpr int kUnitSlack = 6;     // a V tile this far below the accumulators' unit keeps it
+constexpr int kUnitDrop = 72;     // the unit falls at most so far below the largest one passed
 
 // One workgroup: one q head, 4 waves of 16 QT rows each, the K/V tiles of 64
 // rows up to the diagonal.  S^T = K.Q^T and O^T = V^T.P^T, so that a lane's
 // probabilities (one q row, 4 + 4 kv rows per 32) already are the operand of
 // the second product, and the softmax's row factors are one value per lane.  Each
 // product of split operands is three MFMAs (hi.hi + lo.hi + hi.lo; the dropped
-// lo.lo is 2^-22 of a term).  Probabilities are scaled by 2^9 and by the V
-// tile's exponent against the layer's largest, which keeps them in fp16 range
-// and the accumulators in one unit, 2^(vmax - 9); the output's split image
-// takes 2^vmax as its scale (|o| <= the layer's largest |v|).
+// lo.lo is 2^-22 of a term).
+//
+// Exponents.  Probabilities are scaled by 2^9, the accumulators hold the output
+// in units of 2^(unit - 9), and a V tile's exponent against `unit` goes into its
+// probabilities.  Their fp16 pair ends at 2^-25, so `unit` follows a tile that is
+// larger, or smaller by more than 2^6 (which leaves them 2^-28 of a row's largest
+// probability; fp32 has 2^-24 of each), the accumulators rescaled by the exact power
+// of two.  Tiles of one magnitude hardly ever do; one factor for the whole layer would
+// leave the probabilities of a tile 2^-r below the layer's largest 34 - r bits.  Below
+// a tile 2^72 larger the unit stays, or what that tile left in the accumulators
+// could overflow.  The output rows' scale is the largest |v| of any kv head up to
+// the end of their 64-row tile, which bounds |o|: rows to come have no part in it.
 //
 // Iteration t multiplies K tile t + 1, takes tile t through the softmax and
 // multiplies V tile t; the tiles of the next iteration are loaded meanwhile into
 // the other of two buffers each, at one barrier per tile.  One workgroup per CU
 // (128 KB of tiles); the grid's heavy (late) tiles start first and the light ones
-// fill in.  28 layers of 4001 rows: 208 us each (a lone workgroup's tile 2.55 us, one
-// under load 3.15, of which its MFMAs take 1.3 at the nominal clock), 1024 rows 36
-// us.  Measured slower: single-buffered tiles with two workgroups per CU (258 / 43
-// us), two q heads of 64 rows on 8 waves, which reads the LDS twice as much (213 /
-// 48), one MFMA to three VALU instructions enforced (255 / 44).
+// fill in.  Per layer of 4001 rows 202 to 226 us over the boxes, of 1024 rows 35 to
+// 37, of 37 rows 7.3; one exponent for a whole layer took 198 to 223, 34 to 35 and
+// 6.8 on the same ones.  (A lone workgroup's tile takes 2.55 us, one under load 3.15,
+// of which its MFMAs take 1.3 at the nominal clock.)  Measured slower: single-buffered
+// tiles with two workgroups per CU (258 / 43 us), two q heads of 64 rows on 8 waves,
+// which reads the LDS twice as much (213 / 48), one MFMA to three VALU instructions
+// enforced (255 / 44).
 template <int QT>
-__global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L, int layer,
+__global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L,
                                                                    int q_tiles) {
   constexpr int kPlane = kKvTile * kHD * 2;   // bytes of one K or V plane of a tile
   const int lane = lane_id();
@@ -724,6 +732,14 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
   };
   const std::integral_constant<int, 0> b0;
   const std::integral_constant<int, 1> b1;
+  // This wave's rows lie in one 64-row tile, the last whose V rows they see.  The
+  // exponents that bound its output are loaded ahead of everything else and
+  // used at the end (a loop over them here waits for its loads: 1.3 us a workgroup).
+  const int last = min(q0 / kKvTile, tiles - 1), n_exp = (last + 1) * a.Hkv;
+  i32x4 ex[QT];
+#pragma unroll
+  for (int i = 0; i < QT; ++i)
+    ex[i] = *reinterpret_cast<const i32x4*>(a.vexp + min(4 * (kWave * i + lane), (n_exp - 1) & ~3));
   // Q operand: column c = row q0 + 16 i + c, k 8 g .. 8 g + 7 of each 32 dims
   h8 qh[QT][4], ql[QT][4];
   const long qplane = (long)a.Hq * a.S * kHD;
@@ -741,11 +757,11 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
   // scores times that to NaN; other fp16 weights keep it above 2^-76.
   const float fac = fmaxf(
       a.attn_scale * 1.44269504088896340736f * pow2f(head_exp(L.q_norm)) * pow2f(head_exp(L.k_norm)), 0x1p-120f);
-  const int emax = ld_scalar(a.vmax + layer);
-  if (blockIdx.x == 0 && threadIdx.x == 0) a.o_scale[0] = pow2f(emax);
   issue_k(b0, 0);
   issue_v(b0, 0);
   if (nt > 1) issue_k(b1, 1);
+  const int* vexp = a.vexp + kvh;
+  int unit = ld_scalar(vexp), top = unit;
 
   f32x4 o[QT][8];
   float m[QT], l[QT];
@@ -806,9 +822,7 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
   auto body = [&](auto B, auto MORE, int t) {
     constexpr int b = decltype(B)::value;
     const std::integral_constant<int, 1 - b> nb;
-    // probabilities leave exp2 already times 2^ve (V tiles 2^-60 below the
-    // layer's largest vanish in the output's fp16 image, whatever their factor)
-    const int ve = max(ld_scalar(a.vexp + kvh * tiles + t) - emax + kProbExp, -60);
+    const int ev = ld_scalar(vexp + min(t, last) * a.Hkv);   // (past `last` no row sees the tile)
     wait_barrier<0>();   // this iteration's tiles; every wave is done with the buffers refilled below
     if constexpr (decltype(MORE)::value) {
       if (t + 2 < nt) issue_k(B, t + 2);
@@ -843,7 +857,9 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
       mx[i] = fmaxf(v, __shfl_xor(v, 32)) * fac;
       grow = grow || mx[i] > m[i] + kMaxLag;
     }
-    if (__any(grow)) {
+    const int to = ev > unit || ev < unit - kUnitSlack ? max(ev, top - kUnitDrop) : unit;
+    if (to != unit || __any(grow)) {
+      const float f = ldexpf(1.f, unit - to);
 #pragma unroll
       for (int i = 0; i < QT; ++i) {
         const float mn = fmaxf(m[i], mx[i]);
@@ -851,9 +867,13 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
         m[i] = mn;
         l[i] *= al;
 #pragma unroll
-        for (int d = 0; d < 8; ++d) o[i][d] *= al;
+        for (int d = 0; d < 8; ++d) o[i][d] *= al * f;
       }
+      unit = to;
+      top = max(top, to);
     }
+    // probabilities leave exp2 already times 2^ve (2^-60 has them vanish)
+    const int ve = max(ev - unit + kProbExp, -60);
     h8 ph[QT][2], pl[QT][2];
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
@@ -920,13 +940,25 @@ __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const Prefill
     body(b0, end, t);
   }
   const long HD = (long)a.Hq * kHD;
+  int bound = -kMaxExp;
+  auto fold = [&](const i32x4& x, int first) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (first + j < n_exp) bound = max(bound, x[j]);
+  };
+#pragma unroll
+  for (int i = 0; i < QT; ++i) fold(ex[i], min(4 * (kWave * i + lane), (n_exp - 1) & ~3));
+  for (int i = 4 * (kWave * QT + lane); i < n_exp; i += 4 * kWave)
+    fold(*reinterpret_cast<const i32x4*>(a.vexp + i), i);
+  const int o_exp = (int)wave_max((float)bound);
 #pragma unroll
   for (int i = 0; i < QT; ++i) {
     l[i] += __shfl_xor(l[i], 16);
     l[i] += __shfl_xor(l[i], 32);
     const int row = q0 + 16 * i + c;
-    const float inv = 1.f / ((float)(1 << kProbExp) * l[i]);
+    const float inv = ldexpf(1.f / ((float)(1 << kProbExp) * l[i]), unit - o_exp);
     if (row < a.S) {
+      if (head == 0 && g == 0) a.scale[row] = pow2f(o_exp);
       uint16_t* dst = a.img + (long)row * HD + (long)head * kHD + 4 * g;
 #pragma unroll
       for (int d = 0; d < 8; ++d) {
@@ -969,14 +1001,14 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
   const int tiles = (a.S + kKvTile - 1) / kKvTile;
   const int qs = a.Hq * kHD, qn = (a.Hq + 2 * a.Hkv) * kHD;
   int st;
-  const long rot = (long)a.S * (kHD / 2), init = rot > a.layers_n ? rot : a.layers_n;
+  const long init = (long)a.S * (kHD / 2);
   hipLaunchKernelGGL(prefill_init_kernel, dim3((unsigned)((init + 255) / 256)), dim3(256), 0, s, a);
   if ((st = qd_host::launch_status("prefill_init_kernel"))) return st;
   // M rows of the image, whose planes lie `plane` values apart
-  auto gemm = [&](const uint16_t* img, long plane, const uint16_t* W, const float* scale, int scale_stride, int M, int N,
-                  int K, const GemmPlan& g) {
+  auto gemm = [&](const uint16_t* img, long plane, const uint16_t* W, const float* scale, int M, int N, int K,
+                  const GemmPlan& g) {
     SplitGemmArgs x;
-    x.hi = img; x.lo = img + plane; x.scale = scale; x.scale_stride = scale_stride; x.W = W; x.y = a.part;
+    x.hi = img; x.lo = img + plane; x.scale = scale; x.W = W; x.y = a.part;
     x.M = M; x.N = N; x.K = K;
     return split_gemm_launch(x, g, s);
   };
@@ -1000,28 +1032,29 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
     } else if ((st = rows(a.S, p.down[0].z, L.input_norm))) {
       return st;
     }
-    if ((st = gemm(a.img, (long)a.S * a.H, L.qkv, a.scale, 1, a.S, qn, a.H, p.qkv))) return st;
+    if ((st = gemm(a.img, (long)a.S * a.H, L.qkv, a.scale, a.S, qn, a.H, p.qkv))) return st;
     hipLaunchKernelGGL(prefill_qkv_prep_kernel, dim3((unsigned)(qk_groups + a.Hkv * tiles)), dim3(kPrepThreads), 0, s, a,
-                       L, p.qkv.z, qk_groups, li);
+                       L, p.qkv.z, qk_groups);
     if ((st = qd_host::launch_status("prefill_qkv_prep_kernel"))) return st;
     // the last layer's K/V rows are written: past them only the last row is used
     const int last = li + 1 == a.layers_n, M = last ? 1 : a.S;
     const unsigned groups = (unsigned)a.Hq * (last ? 1u : (unsigned)q_tiles);   // last: its final tile
     if (q_rows == 128)
-      hipLaunchKernelGGL((prefill_attention_kernel<2>), dim3(groups), dim3(256), 0, s, a, L, li, q_tiles);
+      hipLaunchKernelGGL((prefill_attention_kernel<2>), dim3(groups), dim3(256), 0, s, a, L, q_tiles);
     else
-      hipLaunchKernelGGL((prefill_attention_kernel<1>), dim3(groups), dim3(256), 0, s, a, L, li, q_tiles);
+      hipLaunchKernelGGL((prefill_attention_kernel<1>), dim3(groups), dim3(256), 0, s, a, L, q_tiles);
     if ((st = qd_host::launch_status("prefill_attention_kernel"))) return st;
-    if ((st = gemm(a.img + (long)(a.S - M) * qs, (long)a.S * qs, L.o_proj, a.o_scale, 0, M, a.H, qs, p.o_proj[last])))
+    if ((st = gemm(a.img + (long)(a.S - M) * qs, (long)a.S * qs, L.o_proj, a.scale + (a.S - M), M, a.H, qs,
+                   p.o_proj[last])))
       return st;
     if ((st = rows(M, p.o_proj[last].z, L.post_norm))) return st;
-    if ((st = gemm(a.img, (long)M * a.H, L.gate_up, a.scale, 1, M, 2 * a.I, a.H, p.gate_up[last]))) return st;
+    if ((st = gemm(a.img, (long)M * a.H, L.gate_up, a.scale, M, 2 * a.I, a.H, p.gate_up[last]))) return st;
     if (M <= qd_host::cu_count())
       hipLaunchKernelGGL(prefill_silu_kernel<1024>, dim3((unsigned)M), dim3(1024), 0, s, a, p.gate_up[last].z);
     else
       hipLaunchKernelGGL(prefill_silu_kernel<256>, dim3((unsigned)M), dim3(256), 0, s, a, p.gate_up[last].z);
     if ((st = qd_host::launch_status("prefill_silu_kernel"))) return st;
-    if ((st = gemm(a.img, (long)M * a.I, L.down, a.scale, 1, M, a.H, a.I, p.down[last]))) return st;
+    if ((st = gemm(a.img, (long)M * a.I, L.down, a.scale, M, a.H, a.I, p.down[last]))) return st;
   }
   return rows(1, p.down[1].z, nullptr);
 }

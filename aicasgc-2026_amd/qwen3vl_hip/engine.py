@@ -12,7 +12,8 @@ Mirrors the reference's decode engine: GreedyDecodeEngine.generate
 (evaluation_wrapper.py:747-1005: static input buffers, graph prebuild and
 replay).  The prefill that fills the static KV cache
 (evaluation_wrapper.py:218-228, a full HF forward in the reference) is one call
-of the native ``qd_prefill`` (fp32 math on the fp16 matrix cores).
+of the native ``qd_prefill`` (activations as two fp16 values on the matrix cores,
+fp32 products and sums).
 """
 
 from __future__ import annotations
@@ -387,12 +388,13 @@ class DecodeEngine(_CapturedSteps):
     # ------------------------------------------------------------ prefill
     @torch.no_grad()
     def prefill(self, prompt: MultimodalPrompt) -> int:
-        """Causal prefill of the prompt into the static cache, in fp32 math.
+        """Causal prefill of the prompt into the static cache.
 
         Follows the text-model loop of transformers Qwen3VLTextModel
         (modeling_qwen3_vl.py:769-852) with M-RoPE positions [3, S]; returns
         the argmax token of the last position.  One call of ``qd_prefill``
-        (HIP kernels) where the library takes the shape, else PyTorch-ROCm ops.
+        (HIP kernels; its header states the precision) where the library takes
+        the shape, else fp32 PyTorch-ROCm ops.
         """
         s = self.shape
         dev = self.device

@@ -505,8 +505,14 @@ int qd_persistent_trace_read(uint64_t* dst, size_t n, int* dims);
  * position_ids (int64 [3][rows], device), causal attention.  Writes cache rows
  * [0, rows) of every layer of d and the greedy token of the last position
  * (first index of the largest fp32 logit) to token_out (device int64 [1]).
- * fp32 math: the fp16 weights meet activations carried as two fp16 values on
- * the matrix cores, at an error no larger than an fp32 GEMM's.  Uses d's
+ * Activations meet the fp16 weights on the matrix cores as two fp16 values of a
+ * common power-of-two scale, 22 bits, products and sums fp32: at N(0, 1) rows the
+ * error is half an fp32 GEMM's.  The values that share a scale are a row (GEMM
+ * inputs), a head (q and k: their norm weights bound them) and 64 rows of one kv
+ * head (V); the attention output's row scale is the largest |v| of any kv head up
+ * to the end of the row's 64-row tile.  Those more than 2^15 below the largest of
+ * them keep an absolute error of 2^-39 of it, where fp32 has 2^-24 of the value.
+ * Rows do not depend on the magnitude of tiles that follow theirs.  Uses d's
  * sizes, weights, inv_freq and caches, not its step state or workspace; the
  * workspace (256-byte aligned, qd_prefill_workspace_bytes bytes, need not be
  * zeroed) is the call's own.  qd_prefill_workspace_bytes returns 0 where the
