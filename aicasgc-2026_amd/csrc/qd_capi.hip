@@ -1321,6 +1321,14 @@ size_t qd_prefill_workspace_bytes(const qd_model_desc* d, int rows) {
 int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int n_vision, const int64_t* text_ids,
                const int64_t* position_ids, int rows, int64_t* token_out, void* workspace, size_t workspace_bytes,
                void* stream) {
+  QD_REQUIRE(d, QD_ERR_ARG, "null pointer");
+  return qd_prefill_layers(d, 0, d->num_layers, vision, vision_dtype, n_vision, text_ids, position_ids, rows, token_out,
+                           workspace, workspace_bytes, stream);
+}
+
+int qd_prefill_layers(const qd_model_desc* d, int first_layer, int n_layers, const void* vision, int vision_dtype,
+                      int n_vision, const int64_t* text_ids, const int64_t* position_ids, int rows, int64_t* token_out,
+                      void* workspace, size_t workspace_bytes, void* stream) {
   QD_REQUIRE(d && d->layers && d->embed && d->final_norm && d->inv_freq && position_ids && token_out && workspace,
              QD_ERR_ARG, "null pointer");
   QD_REQUIRE(vision_dtype == QD_F16 || vision_dtype == QD_F32, QD_ERR_ARG, "bad vision dtype");
@@ -1333,12 +1341,14 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
   const size_t need = prefill_layout(d, rows, &plan, &b);
   QD_REQUIRE(need > 0, QD_ERR_SHAPE, "prefill needs head_dim 128, H in {512, 1024, 2048, 3072, 4096, 6144}, I %% 512 == 0, "
              "Hq %% Hkv == 0 and batch 1");
+  QD_REQUIRE(first_layer >= 0 && n_layers >= 1 && n_layers <= d->num_layers - first_layer, QD_ERR_SHAPE,
+             "layers [%d, %d + %d) of %d", first_layer, first_layer, n_layers, d->num_layers);
   QD_REQUIRE(workspace_bytes >= need && aligned(workspace, 256), QD_ERR_WORKSPACE,
              "workspace of %zu bytes, 256-byte aligned (got %zu)", need, workspace_bytes);
   QD_REQUIRE(a16(d->embed) && a16(d->final_norm), QD_ERR_ARG, "weights must be 16-byte aligned");
-  std::unique_ptr<qd::PrefillLayer[]> layers(new (std::nothrow) qd::PrefillLayer[(size_t)d->num_layers]);
-  QD_REQUIRE(layers, QD_ERR_ARG, "no host memory for %d layers", d->num_layers);
-  for (int i = 0; i < d->num_layers; ++i) {
+  std::unique_ptr<qd::PrefillLayer[]> layers(new (std::nothrow) qd::PrefillLayer[(size_t)n_layers]);
+  QD_REQUIRE(layers, QD_ERR_ARG, "no host memory for %d layers", n_layers);
+  for (int i = first_layer; i < first_layer + n_layers; ++i) {
     const qd_layer_weights& w = d->layers[i];
     QD_REQUIRE(w.qkv && w.o_proj && w.gate_up && w.down && w.input_norm && w.post_norm && w.q_norm && w.k_norm &&
                    w.k_cache && w.v_cache,
@@ -1346,10 +1356,10 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
     QD_REQUIRE(a16(w.qkv) && a16(w.o_proj) && a16(w.gate_up) && a16(w.down) && a16(w.input_norm) && a16(w.post_norm) &&
                    aligned(w.k_cache, 8),
                QD_ERR_ARG, "layer %d: weights must be 16-byte aligned, the K cache 8-byte", i);
-    layers[i] = qd::PrefillLayer{(const u16*)w.qkv,    (const u16*)w.o_proj,     (const u16*)w.gate_up,
-                                 (const u16*)w.down,   (const u16*)w.input_norm, (const u16*)w.post_norm,
-                                 (const u16*)w.q_norm, (const u16*)w.k_norm,     (u16*)w.k_cache,
-                                 (u16*)w.v_cache};
+    layers[i - first_layer] =
+        qd::PrefillLayer{(const u16*)w.qkv,        (const u16*)w.o_proj,    (const u16*)w.gate_up, (const u16*)w.down,
+                         (const u16*)w.input_norm, (const u16*)w.post_norm, (const u16*)w.q_norm,  (const u16*)w.k_norm,
+                         (u16*)w.k_cache,          (u16*)w.v_cache};
   }
   char* base = reinterpret_cast<char*>(workspace);
   qd::PrefillArgs a;
@@ -1368,8 +1378,8 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
   a.vt_img = reinterpret_cast<u16*>(base + b.vt_img);
   a.vexp = reinterpret_cast<int*>(base + b.vexp);
   a.argmax_count = reinterpret_cast<unsigned*>(base + b.argmax);
-  const int st = qd::prefill_launch(a, layers.get(), plan, S(stream));
-  if (st) return st;
+  const int st = qd::prefill_launch(a, layers.get(), first_layer, n_layers, plan, S(stream));
+  if (st || first_layer + n_layers < d->num_layers) return st;
   return qd_lm_head_argmax(a.h + (size_t)(rows - 1) * d->hidden, QD_F32, d->final_norm, d->eps, d->embed, d->vocab,
                            d->hidden, nullptr, token_out, base + b.argmax, stream);
 }

@@ -376,7 +376,9 @@ struct PrefillPlan {
   long part_floats;
 };
 PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I);
-// Every layer; leaves the last row of the residual stream in h.
-int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const PrefillPlan& p, hipStream_t s);
+// Layers [first, first + n), described by layers[0 .. n); the last one leaves the
+// last row of the residual stream in h.
+int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, int first, int n, const PrefillPlan& p,
+                   hipStream_t s);
 
 }  // namespace qd

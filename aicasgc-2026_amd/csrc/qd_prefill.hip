@@ -997,13 +997,16 @@ PrefillPlan prefill_plan(long S, int H, int Hq, int Hkv, int I) {
   return p;
 }
 
-int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const PrefillPlan& p, hipStream_t s) {
+int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, int first, int n, const PrefillPlan& p,
+                   hipStream_t s) {
   const int tiles = (a.S + kKvTile - 1) / kKvTile;
   const int qs = a.Hq * kHD, qn = (a.Hq + 2 * a.Hkv) * kHD;
   int st;
-  const long init = (long)a.S * (kHD / 2);
-  hipLaunchKernelGGL(prefill_init_kernel, dim3((unsigned)((init + 255) / 256)), dim3(256), 0, s, a);
-  if ((st = qd_host::launch_status("prefill_init_kernel"))) return st;
+  if (first == 0) {
+    const long init = (long)a.S * (kHD / 2);
+    hipLaunchKernelGGL(prefill_init_kernel, dim3((unsigned)((init + 255) / 256)), dim3(256), 0, s, a);
+    if ((st = qd_host::launch_status("prefill_init_kernel"))) return st;
+  }
   // M rows of the image, whose planes lie `plane` values apart
   auto gemm = [&](const uint16_t* img, long plane, const uint16_t* W, const float* scale, int M, int N, int K,
                   const GemmPlan& g) {
@@ -1024,8 +1027,8 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
   // 22.5 / 22.0, 3800 27.8 / 26.6)
   const int q_rows = (long)((a.S + 127) / 128) * a.Hq * 4 >= 5L * qd_host::cu_count() ? 128 : 64;
   const int q_tiles = (a.S + q_rows - 1) / q_rows;
-  for (int li = 0; li < a.layers_n; ++li) {
-    const PrefillLayer& L = layers[li];
+  for (int li = first; li < first + n; ++li) {
+    const PrefillLayer& L = layers[li - first];
     if (li == 0) {
       hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((unsigned)a.S), dim3(256), 0, s, a, nullptr, 0, L.input_norm, 0);
       if ((st = qd_host::launch_status("prefill_rows_kernel"))) return st;
@@ -1056,7 +1059,7 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, const Prefi
     if ((st = qd_host::launch_status("prefill_silu_kernel"))) return st;
     if ((st = gemm(a.img, (long)M * a.I, L.down, a.scale, M, a.H, a.I, p.down[last]))) return st;
   }
-  return rows(1, p.down[1].z, nullptr);
+  return first + n == a.layers_n ? rows(1, p.down[1].z, nullptr) : QD_OK;
 }
 
 }  // namespace qd

@@ -19,12 +19,18 @@ fp32 products and sums).
 from __future__ import annotations
 
 import ctypes
+from functools import reduce
+from operator import attrgetter, or_
 
 import torch
 
 from . import _lib
 from .config import QWEN3VL_2B, Qwen3VLTextShape
 from .synthetic import ModelWeights, MultimodalPrompt
+
+_SIZE, _CONTIGUOUS, _DEVICE, _POINTER = (torch.Tensor.size, torch.Tensor.is_contiguous, torch.Tensor.get_device,
+                                         torch.Tensor.data_ptr)
+_DTYPE = attrgetter("dtype")
 
 
 def rope_inv_freq(shape: Qwen3VLTextShape = QWEN3VL_2B) -> torch.Tensor:
@@ -178,12 +184,6 @@ class DecodeEngine(_CapturedSteps):
             L.k_cache = self.k_caches[i].data_ptr()
             L.v_cache = self.v_caches[i].data_ptr()
         self._layers = layers
-        # what the descriptor's raw pointers stand for: the native prefill reads
-        # every weight through them
-        self._native_weights = all(
-            t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0
-            for t in [self.w.embed_tokens, self.w.final_norm_weight] + [t for lw in self.w.layers
-                                                                        for t in lw.tensors().values()])
         d = _lib.ModelDesc()
         d.num_layers = len(self.w.layers)
         d.hidden, d.num_heads, d.num_kv_heads = s.hidden, s.num_heads, s.num_kv_heads
@@ -386,6 +386,28 @@ class DecodeEngine(_CapturedSteps):
             raise RuntimeError("persistent decode step: a workgroup hand-off timed out; results are invalid")
 
     # ------------------------------------------------------------ prefill
+    def _prefill_pointers(self, first: int, n: int):
+        """Addresses of the weights and caches of layers [first, first + n) as the
+        engine holds them now, in LayerDesc's order (their fields may have been
+        rebound or moved since the engine was made), or None where one of them is
+        not what ``qd_prefill`` reads through a pointer."""
+        s, dev = self.shape, self.device.index
+        h, inter, d = s.hidden, s.intermediate, s.head_dim
+        cache = (1, s.num_kv_heads, self.desc.capacity, d)
+        sizes = [(s.qkv_rows, h), (h, s.q_size), (2 * inter, h), (h, inter), (h,), (h,), (d,), (d,), cache, cache] * n
+        ts = []
+        for lw, k, v in zip(self.w.layers[first:first + n], self.k_caches[first:], self.v_caches[first:]):
+            ts += (lw.qkv_weight, lw.o_proj_weight, lw.gate_up_weight, lw.down_proj_weight, lw.input_layernorm_weight,
+                   lw.post_attn_layernorm_weight, lw.q_norm_weight, lw.k_norm_weight, k, v)
+        if first == 0:
+            ts += (self.w.embed_tokens, self.w.final_norm_weight)
+            sizes += [(s.vocab, h), (h,)]
+        if (list(map(_SIZE, ts)) != sizes or set(map(_DTYPE, ts)) != {torch.float16} or set(map(_DEVICE, ts)) != {dev}
+                or not all(map(_CONTIGUOUS, ts))):
+            return None
+        p = list(map(_POINTER, ts))
+        return None if reduce(or_, p) % 16 else p
+
     @torch.no_grad()
     def prefill(self, prompt: MultimodalPrompt) -> int:
         """Causal prefill of the prompt into the static cache.
@@ -405,11 +427,20 @@ class DecodeEngine(_CapturedSteps):
         if ids.numel() and (int(ids.min()) < 0 or int(ids.max()) >= s.vocab):
             raise ValueError(f"prompt token ids outside the vocabulary [0, {s.vocab})")
         lib = _lib.lib()
-        vis, pos = prompt.vision_embeds, prompt.position_ids
-        nbytes = 0
-        if (self._native_weights and vis.ndim == 2 and vis.shape[1] == s.hidden and ids.ndim == 1
-                and tuple(pos.shape) == (3, S) and not pos.is_floating_point()):
-            nbytes = int(lib.qd_prefill_workspace_bytes(ctypes.byref(self.desc), S))
+        vis, pos, inv, n = prompt.vision_embeds, prompt.position_ids, self.inv_freq, len(self.w.layers)
+        # the first layers' pointers, then the others' while the first layers run:
+        # checking all 28 on every call takes the host 0.1 ms
+        head = min(n, 4)
+        nbytes, ptrs = 0, None
+        if (n > 0 and vis.ndim == 2 and vis.shape[1] == s.hidden and ids.ndim == 1 and tuple(pos.shape) == (3, S)
+                and not pos.is_floating_point() and inv.shape == (s.head_dim // 2,) and inv.dtype == torch.float32
+                and inv.get_device() == dev.index and inv.is_contiguous()):
+            ptrs = self._prefill_pointers(0, head)
+        if ptrs is not None:
+            desc, layers = _lib.ModelDesc.from_buffer_copy(self.desc), (ctypes.c_void_p * (10 * n))()
+            desc.num_layers, desc.layers = n, ctypes.cast(layers, ctypes.POINTER(_lib.LayerDesc))
+            desc.inv_freq, desc.final_norm, desc.embed = inv.data_ptr(), ptrs.pop(), ptrs.pop()
+            nbytes = int(lib.qd_prefill_workspace_bytes(ctypes.byref(desc), S))
         if nbytes == 0:
             return self._prefill_general(prompt)
         vis = vis.to(dev)
@@ -419,11 +450,17 @@ class DecodeEngine(_CapturedSteps):
         ids, pos = ids.to(dev, torch.int64).contiguous(), pos.to(dev, torch.int64).contiguous()
         token = torch.empty(1, dtype=torch.int64, device=dev)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
-            _lib.check(lib.qd_prefill(
-                ctypes.byref(self.desc), _lib.ptr(vis), _lib.QD_F32 if vis.dtype == torch.float32 else _lib.QD_F16,
-                int(vis.shape[0]), _lib.ptr(ids), _lib.ptr(pos), S, _lib.ptr(token), _lib.ptr(ws), nbytes,
-                _lib.stream(dev)), "qd_prefill")
+        for first, count in ((0, head), (head, n - head)) if head < n else ((0, n),):
+            if first:
+                ptrs = self._prefill_pointers(first, count)
+                if ptrs is None:
+                    return self._prefill_general(prompt)   # from the start: it writes every cache row again
+            layers[10 * first:10 * (first + count)] = ptrs
+            with torch.cuda.device(dev):
+                _lib.check(lib.qd_prefill_layers(
+                    ctypes.byref(desc), first, count, _lib.ptr(vis),
+                    _lib.QD_F32 if vis.dtype == torch.float32 else _lib.QD_F16, int(vis.shape[0]), _lib.ptr(ids),
+                    _lib.ptr(pos), S, _lib.ptr(token), _lib.ptr(ws), nbytes, _lib.stream(dev)), "qd_prefill_layers")
         return int(token)
 
     def _prefill_general(self, prompt: MultimodalPrompt) -> int:

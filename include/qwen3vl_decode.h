@@ -525,6 +525,15 @@ int qd_prefill(const qd_model_desc* d, const void* vision, int vision_dtype, int
                const int64_t* text_ids, const int64_t* position_ids, int rows, int64_t* token_out,
                void* workspace, size_t workspace_bytes, void* stream);
 
+/* Layers [first_layer, first_layer + n_layers) of a prefill, for a caller that
+ * prepares later layers while earlier ones run: parts in order on one stream,
+ * each with the same prompt and workspace, together equal to qd_prefill.  The
+ * part with the last layer writes token_out.  Only the part's own entries of
+ * d->layers are read. */
+int qd_prefill_layers(const qd_model_desc* d, int first_layer, int n_layers, const void* vision, int vision_dtype,
+                      int n_vision, const int64_t* text_ids, const int64_t* position_ids, int rows,
+                      int64_t* token_out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Synchronously reads the status word of the persistent step, or of the
  * batch step's qkv hand-off (0 = every hand-off completed; bit 0 = a wait
  * exhausted its spin budget, results of that step are invalid) and clears it

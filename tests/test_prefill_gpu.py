@@ -146,3 +146,49 @@ def test_prefill_forms_outside_the_native_route(cuda):
     assert eng.prefill(p) == token and all(torch.equal(a, b) for a, b in zip(k, eng.k_caches))
     with pytest.raises(ValueError):
         eng.prefill(dataclasses.replace(p, text_ids=p.text_ids * 0 + SMALL["vocab"]))
+
+
+@pytest.mark.parametrize("form", ["field", "data", "layer", "embedding", "fp32", "transposed", "cache"])
+@pytest.mark.parametrize("i", [0, 4])
+def test_prefill_reads_the_weights_of_its_call(cuda, form, i):
+    """Weights and caches rebound after the engine was made are the ones used,
+    whatever route their type and layout take; a wrong shape is refused.  The call
+    looks at the first four layers before its first launch, at the others after."""
+    from qwen3vl_hip import synthetic as syn
+    from qwen3vl_hip.config import Qwen3VLTextShape
+    from qwen3vl_hip.engine import DecodeEngine
+
+    shape = Qwen3VLTextShape(num_layers=5, **SMALL)
+    other = syn.model_weights(12, shape, device=cuda)
+    p = syn.multimodal_prompt(11, 1, 2, 3, 9, shape=shape)
+    eng = DecodeEngine(syn.model_weights(11, shape), capacity=p.length + 5)
+    w, held = eng.w, [(lw, lw.down_proj_weight, lw.qkv_weight) for lw in eng.w.layers]   # no old weight is freed
+    held.append((eng.w.embed_tokens, list(eng.k_caches)))
+    first = eng.prefill(p)
+    if form == "field":
+        w.layers[i].down_proj_weight = other.layers[i].down_proj_weight
+    elif form == "data":
+        held.append(w.layers[i].qkv_weight.data)
+        w.layers[i].qkv_weight.data = other.layers[i].qkv_weight
+    elif form == "layer":
+        w.layers[i] = other.layers[i]
+    elif form == "embedding":
+        w.embed_tokens = other.embed_tokens
+    elif form == "fp32":
+        w.layers[i].down_proj_weight = other.layers[i].down_proj_weight.float()
+    elif form == "transposed":
+        w.layers[i].down_proj_weight = other.layers[i].down_proj_weight.T.contiguous().T
+    else:
+        eng.k_caches[i] = torch.zeros_like(eng.k_caches[i])
+    token = eng.prefill(p)
+    _check(w.to("cpu"), p, eng, token)
+    if form == "cache":
+        assert token == first
+    else:
+        fresh = DecodeEngine(w, capacity=eng.capacity)
+        assert fresh.prefill(p) == token
+        for a, b in zip(eng.k_caches + eng.v_caches, fresh.k_caches + fresh.v_caches):
+            assert torch.equal(a, b)
+    w.layers[4 - i].o_proj_weight = w.layers[4 - i].o_proj_weight[:, :-64].contiguous()
+    with pytest.raises(RuntimeError):
+        eng.prefill(p)
