@@ -432,8 +432,10 @@ class DecodeEngine(_CapturedSteps):
         # checking all 28 on every call takes the host 0.1 ms
         head = min(n, 4)
         nbytes, ptrs = 0, None
-        if (n > 0 and vis.ndim == 2 and vis.shape[1] == s.hidden and ids.ndim == 1 and tuple(pos.shape) == (3, S)
-                and not pos.is_floating_point() and inv.shape == (s.head_dim // 2,) and inv.dtype == torch.float32
+        if (n > 0 and vis.ndim == 2 and vis.shape[1] == s.hidden and ids.ndim == 1
+                and ids.dtype in (torch.int64, torch.int32)   # what indexes an embedding: others are refused there
+                and tuple(pos.shape) == (3, S) and not (pos.is_floating_point() or pos.is_complex())
+                and inv.shape == (s.head_dim // 2,) and inv.dtype == torch.float32
                 and inv.get_device() == dev.index and inv.is_contiguous()):
             ptrs = self._prefill_pointers(0, head)
         if ptrs is not None:

@@ -148,6 +148,18 @@ def test_prefill_forms_outside_the_native_route(cuda):
         eng.prefill(dataclasses.replace(p, text_ids=p.text_ids * 0 + SMALL["vocab"]))
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int16, torch.uint8, torch.float32, torch.float64])
+def test_prefill_text_id_types(cuda, dtype):
+    """Ids of a type that does not index an embedding table are refused."""
+    w, p, eng = _run("id types", {**SMALL, "vocab": 200}, (2, 3), 4)
+    q = dataclasses.replace(p, text_ids=p.text_ids.to(dtype))
+    if dtype == torch.int32:
+        assert eng.prefill(q) == eng.prefill(p)
+    else:
+        with pytest.raises(IndexError):
+            eng.prefill(q)
+
+
 @pytest.mark.parametrize("form", ["field", "data", "layer", "embedding", "fp32", "transposed", "cache"])
 @pytest.mark.parametrize("i", [0, 4])
 def test_prefill_reads_the_weights_of_its_call(cuda, form, i):
