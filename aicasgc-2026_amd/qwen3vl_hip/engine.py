@@ -41,18 +41,20 @@ def rope_inv_freq(shape: Qwen3VLTextShape = QWEN3VL_2B) -> torch.Tensor:
 
 
 def _host_ints(x, n: int):
-    """The n values of a flat list, tuple or CPU tensor, or a number, as a
-    ctypes int64 array, or None for anything else (a device tensor stays there,
-    nested and multi-dimensional forms broadcast as torch has it)."""
+    """The n values of a flat list, tuple or CPU tensor of Python ints, or a
+    single one, as a ctypes int64 array, or None for anything else: a device tensor
+    stays there, nested and multi-dimensional forms broadcast as torch has it, and
+    other types and values beyond 64 bits (which ctypes would wrap) convert or are
+    refused as torch does."""
     if torch.is_tensor(x):
         if x.is_cuda or x.ndim != 1:
             return None
         x = x.tolist()
     elif not isinstance(x, (list, tuple)):
         x = [x]
-    if len(x) != n or any(isinstance(v, (list, tuple)) or getattr(v, "shape", ()) != () for v in x):
+    if len(x) != n or not all(isinstance(v, int) and -1 << 63 <= v < 1 << 63 for v in x):
         return None
-    return (ctypes.c_int64 * n)(*(int(v) for v in x))
+    return (ctypes.c_int64 * n)(*x)
 
 
 class _CapturedSteps:
@@ -66,7 +68,7 @@ class _CapturedSteps:
     paid once per replay."""
 
     def _set_state(self, tokens, cache_positions, rope_positions, batch: int, zero_counter: bool) -> bool:
-        """The step state from host values in one launch; False when some are on the device."""
+        """The step state from host values in one launch; False when ``_host_ints`` does not take them."""
         v = [_host_ints(x, batch) for x in (tokens, cache_positions, rope_positions)]
         if any(x is None for x in v):
             return False
@@ -238,7 +240,10 @@ class DecodeEngine(_CapturedSteps):
 
     # ------------------------------------------------------------ state
     def set_state(self, token: int, cache_position: int, rope_position: int) -> None:
-        self._set_state(int(token), int(cache_position), int(rope_position), 1, False)
+        v = int(token), int(cache_position), int(rope_position)
+        if not self._set_state(*v, 1, False):
+            for t, x in zip((self.token, self.cache_position, self.rope_position), v):
+                t.fill_(x)   # raises on the one beyond 64 bits
 
     def reserve_tokens(self, n: int) -> None:
         if self.out_tokens.numel() < n:
@@ -324,7 +329,9 @@ class DecodeEngine(_CapturedSteps):
         if start_position + n_steps > self.capacity:
             raise ValueError("static cache too small for the requested generation")
         self.reserve_tokens(n_steps)
-        self._set_state(int(first_token), int(start_position), int(start_position + rope_delta), 1, True)
+        state = int(first_token), int(start_position), int(start_position + rope_delta)
+        if not self._set_state(*state, 1, True):
+            self.set_state(*state)
         if eos_token_ids is not None and n_steps > 0:
             n_out = self._decode_until_eos(n_steps, use_graph, set(int(t) for t in eos_token_ids),
                                            max(1, int(eos_window)))

@@ -275,3 +275,17 @@ def test_batch_tile_order_layout():
             o8 = ((r // 8) * (K // 64) + k // 64) * 512 + ((k % 64) // 8 % 4) * 128 + ((k % 64) // 32) * 64 \
                 + (r % 8) * 8 + k % 8
             assert t16[o16] == w[r, k] and t8[o8] == w[r, k]
+
+
+def test_host_state_values():
+    """What the one-launch state setter takes as it is; the rest goes to torch's own conversion or refusal."""
+    from qwen3vl_hip.engine import _host_ints
+
+    top = (1 << 63) - 1
+    for x in ([1, -2, top], (1, -2, top), torch.tensor([1, -2, top])):
+        assert list(_host_ints(x, 3)) == [1, -2, top]
+    assert list(_host_ints(-top - 1, 1)) == [-top - 1]
+    for x in ([1, 2, top + 1], [-top - 2, 0, 0], [1, 2], [1, 2, 3.5], [1, 2, "3"], [[1], [2], [3]], [1, 2, None], 5,
+              torch.tensor([1.5, 2, 3]), torch.tensor([[1, 2, 3]]), [1, 2, torch.tensor(3)]):
+        assert _host_ints(x, 3) is None, x
+    assert _host_ints(1 << 64, 1) is None and _host_ints(1.0, 1) is None

@@ -113,3 +113,21 @@ def test_batch_state_forms(cuda, form):
     assert eng.token.tolist() == want[0] and eng.cache_position.tolist() == want[1]
     assert eng.rope_position.tolist() == [[p] * 3 for p in want[2]]
     assert int(eng.step_counter) == 5
+
+
+@pytest.mark.parametrize("bad", [0, 1, 2])
+def test_state_beyond_64_bits_is_refused(cuda, bad):
+    from qwen3vl_hip import synthetic as syn
+    from qwen3vl_hip.config import Qwen3VLTextShape
+    from qwen3vl_hip.engine import BatchDecodeEngine, DecodeEngine
+
+    w = syn.model_weights(3, Qwen3VLTextShape(num_layers=1, vocab=512))
+    v = [1, 2, 3]
+    v[bad] += 1 << 64
+    with pytest.raises((RuntimeError, OverflowError, ValueError)):
+        DecodeEngine(w, 16).set_state(*v)
+    if bad != 1:   # a position is held against the capacity first
+        with pytest.raises((RuntimeError, OverflowError, ValueError)):
+            DecodeEngine(w, 16).decode(v[0], v[1], v[2] - v[1], 1, use_graph=False)
+    with pytest.raises((RuntimeError, OverflowError, ValueError)):
+        BatchDecodeEngine(w, 2, 16).set_state(*([x, x] for x in v))
