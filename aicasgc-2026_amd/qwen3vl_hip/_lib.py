@@ -30,7 +30,6 @@ STEP_AUTO, STEP_CHAIN, STEP_PERSISTENT = 0, 1, 2
 QD_ERR_ARG, QD_ERR_SHAPE = -1, -2
 
 P = c_void_p
-_raw_stream = torch._C._cuda_getCurrentRawStream
 
 # name -> (restype, argtypes)
 _SIGS = {
@@ -126,7 +125,8 @@ def ptr(t: torch.Tensor | None):
 def stream(device: torch.device | None = None) -> int:
     """The current stream of ``device`` (default: the current device) as a pointer."""
     index = None if device is None else device.index
-    return _raw_stream(torch.cuda.current_device() if index is None else index)
+    # looked up here: a torch built without GPU support, which imports this module too, lacks it
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def call(name: str, *args) -> None:

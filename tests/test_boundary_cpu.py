@@ -289,3 +289,13 @@ def test_host_state_values():
               torch.tensor([1.5, 2, 3]), torch.tensor([[1, 2, 3]]), [1, 2, torch.tensor(3)]):
         assert _host_ints(x, 3) is None, x
     assert _host_ints(1 << 64, 1) is None and _host_ints(1.0, 1) is None
+
+
+def test_binding_imports_without_gpu_support_in_torch(monkeypatch):
+    import importlib.util
+
+    from qwen3vl_hip import _lib
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    spec = importlib.util.spec_from_file_location("binding_without_gpu", _lib.__file__)
+    spec.loader.exec_module(importlib.util.module_from_spec(spec))
