@@ -489,7 +489,7 @@ constexpr int kMaxI = 16384;
 // 256 6.8 / 6.1, 300 7.3 / 8.1, 700 10.4 / 12.2, 4001 48.6 (6.1 TB/s) / 59.4.
 template <int NT>
 __global__ __launch_bounds__(NT) void prefill_silu_kernel(const PrefillArgs a, int z) {
-  constexpr int kChunks = kMaxI / (8 * NT);
+  constexpr int kChunks = kMaxI / (8 * NT), kPlanes = NT > 256 ? 4 : 2;
   __shared__ float s_red[NT / kWave];
   const long row = blockIdx.x, n = gridDim.x;
   const long I = a.I;
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(NT) void prefill_silu_kernel(const PrefillArgs a, i
     const long k = (long)c * 8 * NT + threadIdx.x * 8;
     if (k >= I) continue;
     float g[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, p[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll (NT > 256 ? 4 : 2)
+#pragma unroll kPlanes
     for (int i = 0; i < z; ++i) {
       const float* src = a.part + (i * n + row) * 2 * I;
       float v[8], w[8];
