@@ -1384,4 +1384,16 @@ int qd_prefill_layers(const qd_model_desc* d, int first_layer, int n_layers, con
                            d->hidden, nullptr, token_out, base + b.argmax, stream);
 }
 
+int qd_prefill_gemm(const void* hi, const void* lo, const float* scale, const void* W, float* y, int M, int N, int K,
+                    int tile, int z, void* stream) {
+  QD_REQUIRE(hi && lo && scale && W && y, QD_ERR_ARG, "null pointer");
+  QD_REQUIRE(a16(hi) && a16(lo) && a16(W) && a16(y), QD_ERR_ARG, "operands must be 16-byte aligned");
+  qd::SplitGemmArgs a;
+  a.hi = (const u16*)hi; a.lo = (const u16*)lo; a.scale = scale; a.W = (const u16*)W; a.y = y;
+  a.M = M; a.N = N; a.K = K;
+  const int st = qd::split_gemm_launch(a, qd::GemmPlan{tile, z}, S(stream));
+  QD_REQUIRE(st != QD_ERR_SHAPE, QD_ERR_SHAPE, "no tile %d with %d K ranges for %d x %d x %d", tile, z, M, N, K);
+  return st;
+}
+
 }  // extern "C"

@@ -364,7 +364,8 @@ GemmPlan split_gemm_plan(long M, long N, long K) {
 }
 
 int split_gemm_launch(const SplitGemmArgs& a, const GemmPlan& p, hipStream_t s) {
-  if (a.M < 1 || a.N < 4 || a.N % 4 != 0 || p.tile < 0 || p.z < 1 || a.K % kGemmTiles[p.tile].bk != 0 ||
+  constexpr int kTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
+  if (a.M < 1 || a.N < 4 || a.N % 4 != 0 || p.tile < 0 || p.tile >= kTiles || p.z < 1 || p.z > kPrefillMaxSplit || a.K % kGemmTiles[p.tile].bk != 0 ||
       a.K / kGemmTiles[p.tile].bk < p.z)
     return QD_ERR_SHAPE;
   // 32-bit byte offsets into the operands

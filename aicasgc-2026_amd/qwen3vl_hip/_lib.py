@@ -80,6 +80,7 @@ _SIGS = {
     "qd_prefill_workspace_bytes": (c_size_t, [P, c_int]),
     "qd_prefill": (c_int, [P, P, c_int, c_int, P, P, c_int, P, P, c_size_t, P]),
     "qd_prefill_layers": (c_int, [P, c_int, c_int, P, c_int, c_int, P, P, c_int, P, P, c_size_t, P]),
+    "qd_prefill_gemm": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, P]),
     "qd_persistent_trace_read": (c_int, [P, c_size_t, POINTER(c_int)]),
     "qd_batch_gemv_workspace_bytes": (ctypes.c_size_t, [c_long, c_long]),
     "qd_batch_tile_rows": (c_int, [c_long, c_long, c_int]),

@@ -534,6 +534,14 @@ int qd_prefill_layers(const qd_model_desc* d, int first_layer, int n_layers, con
                       int n_vision, const int64_t* text_ids, const int64_t* position_ids, int rows,
                       int64_t* token_out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The prefill's GEMM on its own, with a given tile shape (an index of the tile
+ * table, from 0) and z K ranges (1..16):
+ * y[r][m][n] = scale[m] * sum over K range r of W[n][k] * (hi + lo)[m][k], fp16
+ * operands [M][K] and [N][K] below 4 GB, fp32 y [z][M][N].  QD_ERR_SHAPE where the
+ * tile does not exist or does not divide K into z, or N % 4 != 0. */
+int qd_prefill_gemm(const void* hi, const void* lo, const float* scale, const void* W, float* y, int M, int N,
+                    int K, int tile, int z, void* stream);
+
 /* Synchronously reads the status word of the persistent step, or of the
  * batch step's qkv hand-off (0 = every hand-off completed; bit 0 = a wait
  * exhausted its spin budget, results of that step are invalid) and clears it

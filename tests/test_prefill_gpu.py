@@ -84,6 +84,52 @@ def test_prefill_tile_shapes(cuda, n):
     _run(f"tiles {n}", MODEL, None, n)
 
 
+# Rows, columns and bk of the GEMM's tile table
+GEMM_TILES = [(256, 256, 32), (256, 192, 32), (192, 192, 32), (128, 256, 32), (128, 128, 64), (64, 256, 64),
+              (64, 192, 64), (64, 128, 64), (64, 64, 128), (32, 128, 128), (32, 64, 128), (16, 128, 128)]
+
+
+@pytest.mark.parametrize("tile", range(len(GEMM_TILES)))
+def test_prefill_gemm_tiles(cuda, tile):
+    """Every tile with every K split of the plan, at the edges of its rows, columns
+    and K ranges (one to three blocks, the depth of the ring, and more; ranges of
+    unequal length), so that no plan can choose one that ran nowhere.  An accumulator
+    is rounded some k / 16 times, by 2^-24 of a partial sum that random signs keep
+    below 4 / sqrt(k) of the sum of the products' sizes: sqrt(k) / 4 times 2^-24 of
+    that, and 3 more for short sums, the scale and the planes.  (Without the lo plane:
+    5 times as much at the largest k.)"""
+    from qwen3vl_hip import _lib
+
+    bm, bn, bk = GEMM_TILES[tile]
+    g, worst = torch.Generator().manual_seed(tile), 0.0
+    for z in (1, 2, 3, 4, 6, 8, 12, 16):
+        for m, n, kb in ((1, 4, z), (bm - 1, bn + 4, z + 1), (bm + 1, bn - 4, 2 * z + 1), (2 * bm, 2 * bn, 3 * z),
+                         (2 * bm + 7, bn, 5 * z + max(1, z - 1))):
+            k = kb * bk
+            print(f"case gemm tile {tile} z {z} {m} x {n} x {k}", flush=True)
+            x = torch.randn(m, k, generator=g) * 2.0 ** 12
+            hi = x.half()
+            lo = (x - hi.float()).half()
+            w = torch.randn(n, k, generator=g).mul_(0.02).half()
+            scale = 2.0 ** -torch.randint(0, 20, (m,), generator=g).float()
+            dev = [t.to(cuda) for t in (hi, lo, scale, w)]
+            y = torch.full((z, m, n), float("nan"), device=cuda)
+            _lib.check(_lib.lib().qd_prefill_gemm(dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(),
+                                                  dev[3].data_ptr(), y.data_ptr(), m, n, k, tile, z, _lib.stream(cuda)),
+                       "qd_prefill_gemm")
+            # the reference in 64 bits on the GPU: torch's own product
+            h, l, s, wd = (t.double() for t in dev)
+            ref, size = ((h + l) @ wd.T) * s[:, None], ((h.abs() + l.abs()) @ wd.abs().T) * s[:, None]
+            err = (y.double().sum(0) - ref).abs()
+            assert not bool(err.isnan().any())
+            worst = max(worst, float((err / size).max()) / ((k ** 0.5 / 4 + 3) * 2.0 ** -24))
+            assert worst <= 1, worst
+    print(f"[parity] gemm tile {tile}: worst {worst:.3f} of the bound", flush=True)
+    bad = _lib.lib().qd_prefill_gemm(dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(), dev[3].data_ptr(),
+                                     y.data_ptr(), m, n, bk, tile, 2, _lib.stream(cuda))
+    assert bad == _lib.QD_ERR_SHAPE
+
+
 @pytest.mark.parametrize("n", [2432, 2433, 2560])
 def test_prefill_attention_tile_rows(cuda, n):
     """Both sides of the step from 64 to 128 q rows per attention workgroup (16
