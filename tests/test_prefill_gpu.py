@@ -133,8 +133,15 @@ def test_prefill_gemm_tiles(cuda, tile):
 @pytest.mark.parametrize("n", [2432, 2433, 2560])
 def test_prefill_attention_tile_rows(cuda, n):
     """Both sides of the step from 64 to 128 q rows per attention workgroup (16
-    heads, 256 CUs), and an even multiple of the larger tile."""
-    _run(f"q tiles {n}", MODEL, None, n, layers=1)
+    heads, 256 CUs), and an even multiple of the larger tile; two layers, since the
+    last one runs its last tile alone and the next layer's K/V rows show every row."""
+    _run(f"q tiles {n}", MODEL, None, n)
+
+
+@pytest.mark.parametrize("n", [1152, 1153, 1217, 1345])
+def test_prefill_attention_tile_rows_of_more_heads(cuda, n):
+    """The same step with 32 q heads, and 65 and 1 rows in the last of the larger tiles."""
+    _run(f"q tiles of 32 heads {n}", WIDE, None, n)
 
 
 @pytest.mark.parametrize("grid,n_text", [((3, 5), 1), ((7, 9), 2), ((24, 32), 330), ((40, 44), 351)])
@@ -165,6 +172,14 @@ def test_prefill_rows_far_below_the_rest(cuda, kw, n_text, small):
     lo, hi = small
     _run(f"rows {lo}..{hi} far below, {kw}", kw, (8, 16), n_text, per_row=True,
          scale=lambda n: torch.where((torch.arange(n) >= lo) & (torch.arange(n) < hi), 2.0 ** -36, 1.0))
+
+
+@pytest.mark.parametrize("kw,grid", [(MODEL, (32, 64)), (WIDE, (64, 64))])
+def test_prefill_large_rows_at_the_end(cuda, kw, grid):
+    """The same with the large rows behind more V tiles than a wave's first loads of
+    their exponents cover (256 of 8 heads with 64 q rows, 512 with 128), where a
+    missed one would overflow the last rows."""
+    _run(f"large rows behind {grid}, {kw}", kw, grid, 130, per_row=True, scale=lambda n: torch.full((n,), 2.0 ** -36))
 
 
 @pytest.mark.parametrize("n", [5, 70])
