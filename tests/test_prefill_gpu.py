@@ -46,12 +46,14 @@ def _check(w, prompt, eng, token, per_row=False):
     assert float(logits.max() - logits[token]) <= 1e-4 * float(logits.abs().max())
 
 
+def _not_native(prompt):
+    raise AssertionError("not the native route")
+
+
 def _run(case, shape_kw, grid, n_text, layers=2, scale=None, weights=None, per_row=False):
-    from qwen3vl_hip import _lib, synthetic as syn
+    from qwen3vl_hip import synthetic as syn
     from qwen3vl_hip.config import Qwen3VLTextShape
     from qwen3vl_hip.engine import DecodeEngine
-
-    import ctypes
 
     print(f"case prefill {case}", flush=True)
     shape = Qwen3VLTextShape(num_layers=layers, **shape_kw)
@@ -62,7 +64,7 @@ def _run(case, shape_kw, grid, n_text, layers=2, scale=None, weights=None, per_r
     if scale is not None:
         p = dataclasses.replace(p, vision_embeds=p.vision_embeds.float() * scale(p.vision_embeds.shape[0])[:, None])
     eng = DecodeEngine(w, capacity=p.length + 5)
-    assert _lib.lib().qd_prefill_workspace_bytes(ctypes.byref(eng.desc), p.length) > 0, "not the native route"
+    eng._prefill_general = _not_native
     token = eng.prefill(p)
     _check(w, p, eng, token, per_row)
     before = [t.clone() for t in eng.k_caches + eng.v_caches]
@@ -194,16 +196,19 @@ def test_prefill_forms_outside_the_native_route(cuda):
     their results: the first two by the general path, the last natively."""
     w, p, eng = _run("forms", SMALL, (2, 3), 4)
     token, k = eng.prefill(p), [t.clone() for t in eng.k_caches]
+    general, calls = type(eng)._prefill_general, []
 
-    def again(q):
+    def again(q, native):
         for t in eng.k_caches + eng.v_caches:
             t.zero_()
+        eng._prefill_general = _not_native if native else lambda prompt: calls.append(0) or general(eng, prompt)
+        before = len(calls)
         _check(w, dataclasses.replace(q, position_ids=q.position_ids.long().expand(3, q.length)), eng, eng.prefill(q))
-        return eng
+        assert native or len(calls) == before + 1
 
-    again(dataclasses.replace(p, position_ids=p.position_ids.double()))
-    again(dataclasses.replace(p, position_ids=torch.full((3, 1), 7)))
-    again(dataclasses.replace(p, vision_embeds=p.vision_embeds.double()))
+    again(dataclasses.replace(p, position_ids=p.position_ids.double()), False)
+    again(dataclasses.replace(p, position_ids=torch.full((3, 1), 7)), False)
+    again(dataclasses.replace(p, vision_embeds=p.vision_embeds.double()), True)
     assert eng.prefill(p) == token and all(torch.equal(a, b) for a, b in zip(k, eng.k_caches))
     with pytest.raises(ValueError):
         eng.prefill(dataclasses.replace(p, text_ids=p.text_ids * 0 + SMALL["vocab"]))
@@ -217,6 +222,7 @@ def test_prefill_text_id_types(cuda, dtype):
     if dtype == torch.int32:
         assert eng.prefill(q) == eng.prefill(p)
     else:
+        del eng._prefill_general
         with pytest.raises(IndexError):
             eng.prefill(q)
 
