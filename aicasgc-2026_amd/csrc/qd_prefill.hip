@@ -306,7 +306,8 @@ namespace {
 // per 1024 of K with every CU busy, `idle` of that on an almost idle chip, and
 // the TB/s its loads and stores reach.  Fitted to every shape and K split at
 // 1 .. 4001 rows of the four 2B products (W cold, one workgroup per CU; 4 to 8 %
-// rms, the chosen pair 2.8 % behind the best measured one on average).  The widths
+// rms, the chosen pair 2.8 % behind the best measured one on average); other products
+// and more rows run on what that extrapolates, which nothing measured.  The widths
 // of 192 and the rows below 64 are there for the rounds: 1024 x 12288 x 2048 takes
 // 192 workgroups of 256 x 256 (98 us) or 256 of 256 x 192 (88), 512 rows 58 or 53
 // us; 1300 x 12288 x 2048 148 us on 128 x 128, 134 on 192 x 192.  16 rows of 12288
@@ -680,13 +681,13 @@ constexpr int kUnitDrop = 72;     // the unit falls at most so far below the lar
 // multiplies V tile t; the tiles of the next iteration are loaded meanwhile into
 // the other of two buffers each, at one barrier per tile.  One workgroup per CU
 // (128 KB of tiles); the grid's heavy (late) tiles start first and the light ones
-// fill in.  Per layer of 4001 rows 202 to 226 us over the boxes, of 1024 rows 35 to
-// 37, of 37 rows 7.3; one exponent for a whole layer took 198 to 223, 34 to 35 and
-// 6.8 on the same ones.  (A lone workgroup's tile takes 2.55 us, one under load 3.15,
-// of which its MFMAs take 1.3 at the nominal clock.)  Measured slower: single-buffered
-// tiles with two workgroups per CU (258 / 43 us), two q heads of 64 rows on 8 waves,
-// which reads the LDS twice as much (213 / 48), one MFMA to three VALU instructions
-// enforced (255 / 44).
+// fill in.  Per layer, with one exponent for the whole layer / as it is, us: 4001
+// rows 222 / 226, 1024 rows 35.4 / 36.6, 37 rows 6.8 / 7.3 (boxes differ by 15 %).
+// (A lone workgroup's tile takes 2.55 us, one under load 3.15, of which its MFMAs
+// take 1.3 at the nominal clock.)  Measured slower: single-buffered tiles with two
+// workgroups per CU (258 / 43 us at 4001 / 1024 rows), two q heads of 64 rows on 8
+// waves, which reads the LDS twice as much (213 / 48), one MFMA to three VALU
+// instructions enforced (255 / 44).
 template <int QT>
 __global__ __launch_bounds__(256, 1) void prefill_attention_kernel(const PrefillArgs a, const PrefillLayer L,
                                                                    int q_tiles) {
@@ -1024,8 +1025,8 @@ int prefill_launch(const PrefillArgs& a, const PrefillLayer* layers, int first, 
   const int qk_groups = (int)(((long)a.S * (a.Hq + a.Hkv) + kPrepItems - 1) / kPrepItems);
   // 128 q rows per workgroup read the LDS half as often, 64 give twice the
   // workgroups; they meet at 1.25 workgroups of 128 rows per CU (28 layers of 2B, 64 /
-  // 128 rows: 1800 rows 13.25 / 13.74 ms, 2432 17.50 / 17.64, 2560 18.18 / 18.14, 3000
-  // 22.5 / 22.0, 3800 27.8 / 26.6)
+  // 128 rows: 1800 rows 13.6 / 14.1 ms, 2432 17.98 / 18.10, 2560 18.60 / 18.60, 3000
+  // 22.9 / 22.4, 3800 28.2 / 27.0)
   const int q_rows = (long)((a.S + 127) / 128) * a.Hq * 4 >= 5L * qd_host::cu_count() ? 128 : 64;
   const int q_tiles = (a.S + q_rows - 1) / q_rows;
   for (int li = first; li < first + n; ++li) {
