@@ -682,7 +682,7 @@ constexpr int kUnitDrop = 72;     // the unit falls at most so far below the lar
 // the other of two buffers each, at one barrier per tile.  One workgroup per CU
 // (128 KB of tiles); the grid's heavy (late) tiles start first and the light ones
 // fill in.  Per layer, with one exponent for the whole layer / as it is, us: 4001
-// rows 222 / 226, 1024 rows 35.4 / 36.6, 37 rows 6.8 / 7.3 (boxes differ by 15 %).
+// rows 222 / 226, 1024 rows 35.4 / 36.6, 37 rows 6.8 / 7.3 (cards differ by 15 %).
 // (A lone workgroup's tile takes 2.55 us, one under load 3.15, of which its MFMAs
 // take 1.3 at the nominal clock.)  Measured slower: single-buffered tiles with two
 // workgroups per CU (258 / 43 us at 4001 / 1024 rows), two q heads of 64 rows on 8

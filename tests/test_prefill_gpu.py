@@ -271,3 +271,33 @@ def test_prefill_reads_the_weights_of_its_call(cuda, form, i):
     w.layers[4 - i].o_proj_weight = w.layers[4 - i].o_proj_weight[:, :-64].contiguous()
     with pytest.raises(RuntimeError):
         eng.prefill(p)
+
+
+@pytest.mark.parametrize("cuts", [(0, 5), (0, 1, 5), (0, 2, 4, 5)])
+def test_prefill_in_parts(cuda, cuts):
+    """The C entries: a whole prefill and one in parts, bit for bit the engine's (whose
+    own parts are of four layers and the rest), with a workspace full of NaN."""
+    import ctypes
+
+    from qwen3vl_hip import _lib
+
+    w, p, eng = _run(f"parts {cuts}", SMALL, (2, 3), 70, layers=5)
+    token, before = eng.prefill(p), [t.clone() for t in eng.k_caches + eng.v_caches]
+    for t in eng.k_caches + eng.v_caches:
+        t.zero_()
+    lib, d, n = _lib.lib(), ctypes.byref(eng.desc), p.length
+    nbytes = lib.qd_prefill_workspace_bytes(d, n)
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=cuda)
+    out = torch.full((1,), -1, dtype=torch.int64, device=cuda)
+    vis, ids, pos = (t.to(cuda).contiguous() for t in (p.vision_embeds, p.text_ids, p.position_ids))
+    args = (vis.data_ptr(), _lib.QD_F16, vis.shape[0], ids.data_ptr(), pos.data_ptr(), n, out.data_ptr(), ws.data_ptr(),
+            nbytes, _lib.stream(cuda))
+    for first, count in ((-1, 2), (0, 0), (0, 6), (5, 1), (4, 2)):
+        assert lib.qd_prefill_layers(d, first, count, *args) == _lib.QD_ERR_SHAPE
+    if len(cuts) == 2:
+        _lib.check(lib.qd_prefill(d, *args), "qd_prefill")
+    for a, b in zip(cuts, cuts[1:]) if len(cuts) > 2 else ():
+        assert int(out) == -1
+        _lib.check(lib.qd_prefill_layers(d, a, b - a, *args), "qd_prefill_layers")
+    assert int(out) == token
+    assert all(torch.equal(a, b) for a, b in zip(before, eng.k_caches + eng.v_caches))
